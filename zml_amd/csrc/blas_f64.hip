@@ -1,14 +1,6 @@
-// Level-1/2/3 helpers on the device: TRSM and SYRK (FP64 and FP32), IDAMAX,
+// Level-1/2/3 helpers on the device: SYRK (FP64 and FP32), IDAMAX,
 // DSCAL, DSWAP, row interchanges (LASWP), transposes, GEMV, TRSV and the
 // matrix norms of LANGE.
-//
-// TRSM is blocked: 32 x 32 diagonal blocks are solved by substitution (one
-// thread per right-hand-side vector, the block staged in LDS), and the rest
-// of the right-hand sides are updated with the MFMA GEMM. The arithmetic
-// choices follow zml's trsm.zig where they are visible in a result: the
-// left-side branches divide by the diagonal (trsm.zig:137-142,221-229,
-// 298-305,364-371), the right-side branches multiply by its reciprocal
-// (trsm.zig:458-486,538-566,575-600,653-678).
 #include "zmlhip_internal.hpp"
 
 #include <algorithm>
@@ -16,62 +8,6 @@
 
 namespace zmlhip {
 namespace {
-
-constexpr int TB = 32;   // diagonal block size of the blocked TRSM
-
-// Solves M x = b for each vector x of a 32-row block (left side: vectors are
-// columns of B; right side: rows of B, with M the transpose of op(T)), in the
-// column-sweep order of zml's no-transpose loops.
-// forward: M lower (k ascending); else M upper (k descending).
-template <typename T, bool LEFT>
-__global__ void __launch_bounds__(256)
-trsm_diag_kernel(int nb, const T* __restrict__ a, int64_t lda, int need_t, int forward,
-                 int unit, T* __restrict__ b, int64_t ldb, int64_t nvec) {
-  // separately rounded multiply and subtract, as zml's substitution loops
-  // (trsm.zig, trsv.zig): exact cancellations stay exact
-#pragma clang fp contract(off)
-  __shared__ T M[TB][TB + 1];
-  __shared__ T dinv[TB];
-  for (int e = threadIdx.x; e < TB * TB; e += blockDim.x) {
-    const int r = e % TB, c = e / TB;
-    T v = T(0);
-    if (r < nb && c < nb) v = need_t ? a[c + (int64_t)r * lda] : a[r + (int64_t)c * lda];
-    M[r][c] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < TB) dinv[threadIdx.x] = threadIdx.x < nb ? T(1) / M[threadIdx.x][threadIdx.x] : T(1);
-  __syncthreads();
-  const int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (v >= nvec) return;
-  T x[TB];
-#pragma unroll
-  for (int r = 0; r < TB; ++r) x[r] = r < nb ? (LEFT ? b[r + v * ldb] : b[v + (int64_t)r * ldb]) : T(0);
-  if (forward) {
-#pragma unroll
-    for (int k = 0; k < TB; ++k) {
-      if (k < nb) {
-        if (!unit) x[k] = LEFT ? x[k] / M[k][k] : x[k] * dinv[k];
-#pragma unroll
-        for (int i = k + 1; i < TB; ++i) x[i] -= x[k] * M[i][k];
-      }
-    }
-  } else {
-#pragma unroll
-    for (int k = TB - 1; k >= 0; --k) {
-      if (k < nb) {
-        if (!unit) x[k] = LEFT ? x[k] / M[k][k] : x[k] * dinv[k];
-#pragma unroll
-        for (int i = 0; i < k; ++i) x[i] -= x[k] * M[i][k];
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < TB; ++r)
-    if (r < nb) {
-      if (LEFT) b[r + v * ldb] = x[r];
-      else b[v + (int64_t)r * ldb] = x[r];
-    }
-}
 
 // ---- IDAMAX: first index of max |x| (iamax.zig:11-68; NaN never wins unless x[0] is NaN)
 struct AmaxPair { double v; int64_t i; };
@@ -230,62 +166,6 @@ inline int grid_for(int64_t n, int threads = 256, int cap = 65536) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
-template <typename T>
-void trsm_cm(int side, int uplo, int transa, int diag, int64_t m, int64_t n, T alpha, const T* a,
-             int64_t lda, T* b, int64_t ldb, hipStream_t s) {
-  if (m <= 0 || n <= 0) return;
-  if (alpha == T(0)) { scale_cm<T>(m, n, T(0), b, ldb, s, 0); return; }   // trsm.zig:99-113
-  if (alpha != T(1)) scale_cm<T>(m, n, alpha, b, ldb, s, 0);
-  const bool nt = is_notrans(transa);
-  const bool unit = diag == kUnit;
-  if (side == kLeft) {
-    // op(A) is m x m; solve op(A) X = B block row by block row.
-    const bool fwd = (uplo == kLower) == nt;   // op(A) lower -> forward
-    const int64_t nblk = (m + TB - 1) / TB;
-    for (int64_t bi = 0; bi < nblk; ++bi) {
-      const int64_t blk = fwd ? bi : nblk - 1 - bi;
-      const int64_t i0 = blk * TB, nb = std::min<int64_t>(TB, m - i0);
-      hipLaunchKernelGGL((trsm_diag_kernel<T, true>), dim3(grid_for(n)), dim3(256), 0, s, (int)nb,
-                         a + i0 + i0 * lda, lda, nt ? 0 : 1, fwd ? 1 : 0, unit ? 1 : 0,
-                         b + i0, ldb, n);
-      ZH_LAUNCH_CHECK();
-      // update the remaining rows: B_rest -= op(A)_{rest, blk} X_blk
-      const int64_t r0 = fwd ? i0 + nb : 0, rn = fwd ? m - (i0 + nb) : i0;
-      if (rn > 0) {
-        if (nt) gemm_cm<T>(kNoTrans, kNoTrans, rn, n, nb, T(-1), a + r0 + i0 * lda, lda, b + i0, ldb, T(1), b + r0, ldb, s, 0);
-        else gemm_cm<T>(kTrans, kNoTrans, rn, n, nb, T(-1), a + i0 + r0 * lda, lda, b + i0, ldb, T(1), b + r0, ldb, s, 0);
-      }
-    }
-  } else {
-    // X op(A) = B with op(A) n x n, block column by block column.
-    const bool fwd = (uplo == kUpper) == nt;   // op(A) upper -> X_j depends on X_<j
-    const int64_t nblk = (n + TB - 1) / TB;
-    for (int64_t bj = 0; bj < nblk; ++bj) {
-      const int64_t blk = fwd ? bj : nblk - 1 - bj;
-      const int64_t j0 = blk * TB, nb = std::min<int64_t>(TB, n - j0);
-      // rows of B solve x M = b, i.e. M^T x^T = b^T with M = op(A_jj)
-      hipLaunchKernelGGL((trsm_diag_kernel<T, false>), dim3(grid_for(m)), dim3(256), 0, s, (int)nb,
-                         a + j0 + j0 * lda, lda, nt ? 1 : 0, fwd ? 1 : 0, unit ? 1 : 0,
-                         b + j0 * ldb, ldb, m);
-      ZH_LAUNCH_CHECK();
-      const int64_t c0 = fwd ? j0 + nb : 0, cn = fwd ? n - (j0 + nb) : j0;
-      if (cn > 0) {
-        if (nt) gemm_cm<T>(kNoTrans, kNoTrans, m, cn, nb, T(-1), b + j0 * ldb, ldb, a + j0 + c0 * lda, lda, T(1), b + c0 * ldb, ldb, s, 0);
-        else gemm_cm<T>(kNoTrans, kTrans, m, cn, nb, T(-1), b + j0 * ldb, ldb, a + c0 + j0 * lda, lda, T(1), b + c0 * ldb, ldb, s, 0);
-      }
-    }
-  }
-}
-template void trsm_cm<double>(int, int, int, int, int64_t, int64_t, double, const double*, int64_t, double*,
-                              int64_t, hipStream_t);
-template void trsm_cm<float>(int, int, int, int, int64_t, int64_t, float, const float*, int64_t, float*,
-                             int64_t, hipStream_t);
-
-void trsm_f64_cm(int side, int uplo, int transa, int diag, int64_t m, int64_t n, double alpha,
-                 const double* a, int64_t lda, double* b, int64_t ldb, hipStream_t s) {
-  trsm_cm<double>(side, uplo, transa, diag, m, n, alpha, a, lda, b, ldb, s);
-}
-
 template <typename T>
 void syrk_cm(int uplo, int trans, int64_t n, int64_t k, T alpha, const T* a, int64_t lda, T beta, T* c,
              int64_t ldc, hipStream_t s) {
