@@ -27,34 +27,181 @@ namespace {
 
 constexpr int DB = 128;   // diagonal block of the driver
 
-// Unblocked Cholesky of an nb x nb block (nb <= DB), register resident.
+// Cholesky of an nb x nb block (nb <= DB) by one workgroup, register resident.
 // lower: A = L L^T on the lower triangle; else A = U^T U on the upper one.
-// Thread (tx, ty) of a 16 x 16 grid holds the elements (tx + 16 ii, ty + 16 cc),
-// ii >= cc, of the lower-orientation block in registers. Column j travels
-// through LDS unscaled (double buffered, one barrier per column); every thread
-// takes l_jj = sqrt(a_jj), r = fl(1 / l_jj) and l_ij = fl(a_ij * r) from it, so
-// the trailing update a_ic - l_ij * l_cj uses the same separately rounded
-// values, in the same right-looking order, as the unblocked algorithm.
-__device__ __forceinline__ double sqrt_rn(double x) { return sqrt(x); }   // IEEE, correctly rounded
-__device__ __forceinline__ float sqrt_rn(float x) { return sqrtf(x); }
+// A 16 x 16 thread grid holds the elements (i + 16 ii, c + 16 cc), ii >= cc, of
+// the lower-orientation block. The block advances in chunks of 16 columns:
+//   the chunk goes to LDS;
+//   up to three waves factor it, one row per lane with its 16 values in
+//   registers: lanes 0..15 of every wave hold the chunk's own 16 rows (the same
+//   values in each wave, so no step needs a barrier), lanes 16..63 the rows
+//   below. A step takes l_jj = sqrt(a_jj) and r = fl(1 / l_jj) from lane j,
+//   l_ij = fl(a_ij r), and the other chunk rows' multipliers by readlane;
+//   every thread applies the chunk's 16 columns to its later columns, from LDS.
+// Each element receives its separately rounded updates a - l_ik l_ck in the order
+// of k, as in the unblocked right-looking algorithm: the same bits as one column
+// at a time over the whole block, which spent its time on masks and on one
+// barrier per column (158 us per 128 x 128 block on MI355X, against 42 us). Bound by
+// the step chain of one wave (310 cycles a column: square root, reciprocal, up to
+// 15 readlane pairs with their multiplies and subtracts), then by the later
+// columns' updates (230 cycles a column on average).
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)u, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(u >> 32), lane);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// l = sqrt(d), r = fl(1 / l), both correctly rounded. FP64: Goldschmidt's iteration
+// from the hardware's reciprocal square root with two residual corrections of
+// the root, whose half reciprocal then starts Newton's iteration for 1 / l (two
+// corrections, Markstein): 100 cycles against 175 for sqrt and a division. Both
+// of those outside [2^-512, 2^512); d must be the same in every lane. False, with
+// l = r = 1, where d is not positive.
+__device__ __forceinline__ bool sqrt_and_inv(double d, double& l, double& r) {
+  const uint32_t hi = (uint32_t)((uint64_t)__double_as_longlong(d) >> 32);
+  constexpr uint32_t kLow = (1023u - 512u) << 20, kSpan = 1024u << 20;
+  if (__builtin_expect(hi - kLow < kSpan, 1)) {
+    const double y = __builtin_amdgcn_rsq(d);
+    double g = d * y, h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, d), h, g);
+    g = fma(fma(-g, g, d), h, g);
+    double z = h + h;
+    z = fma(fma(-g, z, 1.0), z, z);
+    z = fma(fma(-g, z, 1.0), z, z);
+    // a root with every mantissa bit set is the one divisor whose reciprocal the
+    // corrections leave one bit low (2^-k where 2^-k (1 + 2^-52) is nearest)
+    constexpr uint64_t kMant = 0xfffffffffffffull;
+    const uint64_t ones = ((uint64_t)__double_as_longlong(g) & kMant) == kMant ? 1u : 0u;
+    l = g;
+    r = __longlong_as_double((long long)((uint64_t)__double_as_longlong(z) | ones));
+    return true;
+  }
+  const bool ok = d > 0.0;
+  l = ok ? sqrt(d) : 1.0;
+  r = 1.0 / l;
+  return ok;
+}
+__device__ __forceinline__ bool sqrt_and_inv(float d, float& l, float& r) {
+  const bool ok = d > 0.0f;
+  l = ok ? sqrtf(d) : 1.0f;
+  r = 1.0f / l;
+  return ok;
+}
+
+constexpr int CW = 16;         // columns of a chunk
+constexpr int PLD = CW + 1;    // LDS row stride of a chunk
+
+// Step J of a chunk on one row per lane (p: its 16 values).
+template <typename T, int J>
+__device__ __forceinline__ void chunk_steps(T (&p)[CW], int lane, int j0, int& fail) {
+#pragma clang fp contract(off)
+  if constexpr (J < CW) {
+    T ljj, rj;
+    if (!sqrt_and_inv(lane_value(p[J], J), ljj, rj) && !fail) fail = j0 + J + 1;
+    const T l = p[J] * rj;
+    p[J] = lane == J ? ljj : l;
+    // four columns at a time: their multipliers, the products, the subtractions
+    // (one after the other each column would wait for its own chain)
+#pragma unroll
+    for (int c = J + 1; c < CW; c += 4) {
+      T m[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m[e] = c + e < CW ? lane_value(l, c + e < CW ? c + e : 0) : T(0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < CW) m[e] = l * m[e];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < CW) p[c + e] = p[c + e] - m[e];
+    }
+    chunk_steps<T, J + 1>(p, lane, j0, fail);
+  }
+}
+
+// Chunk CH of the thread's elements to LDS; the factored chunk back, and its 16
+// columns, in order, into the thread's later columns.
+template <typename T, int CH>
+__device__ __forceinline__ void chunk_out(const T (&v)[8][8], T* P, int ri, int ci) {
+#pragma unroll
+  for (int ii = CH; ii < 8; ++ii) P[(ri + 16 * ii) * PLD + ci] = v[ii][CH];
+}
+template <typename T, int CH>
+__device__ __forceinline__ void chunk_apply(T (&v)[8][8], const T* R, int ri, int ci) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int ii = CH; ii < 8; ++ii) v[ii][CH] = R[(ri + 16 * ii) * PLD + ci];
+  if constexpr (CH < 7) {
+#pragma unroll 4
+    for (int k = 0; k < CW; ++k) {
+      T lr[8], lc[8];
+#pragma unroll
+      for (int ii = CH + 1; ii < 8; ++ii) {
+        lr[ii] = R[(ri + 16 * ii) * PLD + k];
+        lc[ii] = R[(ci + 16 * ii) * PLD + k];
+      }
+#pragma unroll
+      for (int ii = CH + 1; ii < 8; ++ii)
+#pragma unroll
+        for (int cc = CH + 1; cc <= ii; ++cc) v[ii][cc] = v[ii][cc] - lr[ii] * lc[cc];
+    }
+  }
+}
+template <typename T>
+__device__ __forceinline__ void chunk_out(int ch, const T (&v)[8][8], T* P, int ri, int ci) {
+  switch (ch) {
+    case 0: chunk_out<T, 0>(v, P, ri, ci); break;
+    case 1: chunk_out<T, 1>(v, P, ri, ci); break;
+    case 2: chunk_out<T, 2>(v, P, ri, ci); break;
+    case 3: chunk_out<T, 3>(v, P, ri, ci); break;
+    case 4: chunk_out<T, 4>(v, P, ri, ci); break;
+    case 5: chunk_out<T, 5>(v, P, ri, ci); break;
+    case 6: chunk_out<T, 6>(v, P, ri, ci); break;
+    default: chunk_out<T, 7>(v, P, ri, ci); break;
+  }
+}
+template <typename T>
+__device__ __forceinline__ void chunk_apply(int ch, T (&v)[8][8], const T* R, int ri, int ci) {
+  switch (ch) {
+    case 0: chunk_apply<T, 0>(v, R, ri, ci); break;
+    case 1: chunk_apply<T, 1>(v, R, ri, ci); break;
+    case 2: chunk_apply<T, 2>(v, R, ri, ci); break;
+    case 3: chunk_apply<T, 3>(v, R, ri, ci); break;
+    case 4: chunk_apply<T, 4>(v, R, ri, ci); break;
+    case 5: chunk_apply<T, 5>(v, R, ri, ci); break;
+    case 6: chunk_apply<T, 6>(v, R, ri, ci); break;
+    default: chunk_apply<T, 7>(v, R, ri, ci); break;
+  }
+}
 
 template <typename T>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 1)
 potrf_diag_kernel(int nb, T* __restrict__ a, int64_t lda, int lower, int* __restrict__ info,
                   int64_t info_base) {
-#pragma clang fp contract(off)
-  __shared__ T colbuf[2][DB];
+  __shared__ T P[DB * PLD], R[DB * PLD];   // the chunk before and after its 16 steps
+  __shared__ int s_fail;
   if (*info != 0) return;   // an earlier block already failed
-  const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  // memory's contiguous direction runs along the low 4 bits of the thread index
+  const int ri = lower ? t & 15 : t >> 4, ci = lower ? t >> 4 : t & 15;
+  if (t == 0) s_fail = 0;
   T v[8][8];
   // every address of the nb x nb block is readable: all 36 loads are issued
   // unconditionally (clamped indices; the empty asm keeps the compiler from
-  // sinking each one under its mask and waiting for it), then masked
+  // sinking each one under its mask and waiting for it), then masked; rows from nb
+  // on are those of the identity
 #pragma unroll
   for (int ii = 0; ii < 8; ++ii)
 #pragma unroll
     for (int cc = 0; cc <= ii; ++cc) {
-      const int r = tx + 16 * ii, c = ty + 16 * cc;
+      const int r = ri + 16 * ii, c = ci + 16 * cc;
       const int64_t rc = r < nb ? r : nb - 1, cl = c < nb ? c : nb - 1;
       v[ii][cc] = a[lower ? rc + cl * lda : cl + rc * lda];
     }
@@ -63,73 +210,46 @@ potrf_diag_kernel(int nb, T* __restrict__ a, int64_t lda, int lower, int* __rest
 #pragma unroll
     for (int cc = 0; cc <= ii; ++cc) {
       asm volatile("" : "+v"(v[ii][cc]));
-      const int r = tx + 16 * ii, c = ty + 16 * cc;
-      if (!(r < nb && c <= r)) v[ii][cc] = T(0);
+      const int r = ri + 16 * ii, c = ci + 16 * cc;
+      if (!(r < nb && c <= r)) v[ii][cc] = r == c ? T(1) : T(0);
     }
-  // column 0 (ty == 0, cc == 0)
-  if (ty == 0) {
+
+  const int nch = (nb + CW - 1) / CW;
+  int done = nb;   // columns that were completed
+  for (int ch = 0; ch < nch; ++ch) {
+    const int j0 = CW * ch;
+    chunk_out<T>(ch, v, P, ri, ci);
+    __syncthreads();
+    // the chunk's 16 columns: rows j0 .. j0 + 15 in every wave's lanes 0..15
+    const int row = lane < CW ? j0 + lane : j0 + CW + (64 - CW) * w + lane - CW;
+    if (w == 0 || j0 + CW + (64 - CW) * w < nb) {
+      T p[CW];
+      const int rl = row < DB ? row : DB - 1;
 #pragma unroll
-    for (int ii = 0; ii < 8; ++ii)
-      if (tx + 16 * ii < nb) colbuf[0][tx + 16 * ii] = v[ii][0];
-  }
-  __syncthreads();
-  int fail = 0;
-  for (int j = 0; j < nb; ++j) {
-    const T* cur = colbuf[j & 1];
-    const T d = cur[j];
-    if (!(d > T(0))) { fail = j + 1; break; }   // non-positive or NaN pivot
-    const T ljj = sqrt_rn(d);
-    const T rj = T(1) / ljj;
-    T lr[8], lc[8];
+      for (int c = 0; c < CW; ++c) p[c] = P[rl * PLD + c];
+      int fail = 0;
+      chunk_steps<T, 0>(p, lane, j0, fail);
+      if (lane >= CW ? row < DB : w == 0) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      lr[k] = cur[tx + 16 * k] * rj;
-      lc[k] = cur[ty + 16 * k] * rj;
-    }
-    const int jc = j >> 4, jt = j & 15;
-#pragma unroll
-    for (int cc = 0; cc < 8; ++cc) {
-      if (cc == jc && ty == jt) {   // this thread holds part of column j: finalize it
-#pragma unroll
-        for (int ii = cc; ii < 8; ++ii) {
-          const int r = tx + 16 * ii;
-          if (r == j) v[ii][cc] = ljj;
-          else if (r > j) v[ii][cc] = lr[ii];
-        }
+        for (int c = 0; c < CW; ++c) R[rl * PLD + c] = p[c];
       }
-      if (16 * cc + 15 > j) {   // some column of this group lies right of j
-        const int c = ty + 16 * cc;
-#pragma unroll
-        for (int ii = cc; ii < 8; ++ii) {
-          const int r = tx + 16 * ii;
-          if (c > j && c <= r && r < nb) v[ii][cc] = v[ii][cc] - lr[ii] * lc[cc];
-        }
-      }
-    }
-    // publish column j + 1, now fully updated
-    const int jn = j + 1;
-    if (jn < nb && ty == (jn & 15)) {
-#pragma unroll
-      for (int cc = 0; cc < 8; ++cc)
-        if (cc == (jn >> 4)) {
-#pragma unroll
-          for (int ii = cc; ii < 8; ++ii) {
-            const int r = tx + 16 * ii;
-            if (r >= jn && r < nb) colbuf[jn & 1][r] = v[ii][cc];
-          }
-        }
+      if (fail && w == 0 && lane == 0) s_fail = fail;
     }
     __syncthreads();
+    chunk_apply<T>(ch, v, R, ri, ci);
+    if (s_fail) {   // (s_fail only changes between this and the next barrier's far side)
+      done = s_fail - 1;
+      break;
+    }
   }
-  const int done = fail ? fail - 1 : nb;   // columns that were completed
 #pragma unroll
   for (int ii = 0; ii < 8; ++ii)
 #pragma unroll
     for (int cc = 0; cc <= ii; ++cc) {
-      const int r = tx + 16 * ii, c = ty + 16 * cc;
+      const int r = ri + 16 * ii, c = ci + 16 * cc;
       if (r < nb && c <= r && c < done) a[lower ? r + (int64_t)c * lda : c + (int64_t)r * lda] = v[ii][cc];
     }
-  if (fail && t == 0) *info = (int)(info_base + fail);
+  if (done < nb && t == 0) *info = (int)(info_base + done + 1);
 }
 
 }  // namespace
