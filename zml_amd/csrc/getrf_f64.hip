@@ -23,6 +23,7 @@
 #include "zmlhip_internal.hpp"
 #include "panel.hpp"
 #include "panel_fused.hpp"
+#include "panel_leaf1.hpp"
 #include "mixed.hpp"
 
 #include <algorithm>
@@ -61,7 +62,7 @@ static LeafState& leaf_state(hipStream_t s, void** ws_out) {
     int per_cu = 0;
     int per_cu_la = 0;
     ZH_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, panel::leaf_kernel<double, true>, panel::pt_of<double>(), 0));
+        &per_cu, panel::leaf_kernel<double>, panel::pt_of<double>(), 0));
     ZH_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu_la, panel::leaf_la_kernel<double>, panel::la_threads<double>(), 0));
     st.max_resident = std::max(1, std::min(per_cu, per_cu_la)) * device_cu_count();
@@ -71,35 +72,57 @@ static LeafState& leaf_state(hipStream_t s, void** ws_out) {
 }
 
 // Factor one leaf (rows [r0, m), columns [c0, c0 + w)) of a row-major matrix.
+// Up to kLeaf1Rows rows go to one workgroup, which also writes the leaf's row
+// moves into `moves` (true); more are spread over workgroups that exchange every
+// pivot through memory, and the caller composes the moves from ipiv (false).
+// The line: 1,024 rows are what a workgroup's registers hold (512 threads, two
+// rows each, 32 columns at a time). At that height the one-workgroup leaf takes
+// 152 us, four exchanging workgroups 320 us (MI355X, FP64). A forced give-up of the
+// exchange (negative spin limit) takes the exchanging leaf as far as it goes.
+constexpr int64_t kLeaf1Rows = 1024;
 template <typename T>
-void leaf_factor(int64_t m, T* A, int64_t lda, int64_t r0, int64_t c0, int w, int32_t* ipiv,
-                 int* info, hipStream_t s) {
-  void* ws = nullptr;
-  LeafState& st = leaf_state(s, &ws);
+bool leaf_factor(int64_t m, T* A, int64_t lda, int64_t r0, int64_t c0, int w, int32_t* ipiv,
+                 int* info, int32_t* moves, hipStream_t s) {
   const int64_t M = m - r0;
   constexpr int PT = panel::pt_of<T>();
+  if (M <= (panel_spin_limit() < 0 ? (int64_t)PT : kLeaf1Rows)) {
+    T* const p = A + r0 * lda + c0;
+    constexpr int HW = sizeof(T) == 8 ? 32 : 64;   // columns of the two-rows-per-thread form
+    if (M <= 64)
+      hipLaunchKernelGGL((panel::leaf1_kernel<T, 64, 1, 64>), dim3(1), dim3(64), 0, s, (int)M, w, p, lda, ipiv + r0,
+                         r0, info, c0, moves);
+    else if (M <= 256)
+      hipLaunchKernelGGL((panel::leaf1_kernel<T, 256, 1, 64>), dim3(1), dim3(256), 0, s, (int)M, w, p, lda,
+                         ipiv + r0, r0, info, c0, moves);
+    else if (M <= 512)
+      hipLaunchKernelGGL((panel::leaf1_kernel<T, 512, 1, 64>), dim3(1), dim3(512), 0, s, (int)M, w, p, lda,
+                         ipiv + r0, r0, info, c0, moves);
+    else
+      hipLaunchKernelGGL((panel::leaf1_kernel<T, 512, 2, HW>), dim3(1), dim3(512), 0, s, (int)M, w, p, lda,
+                         ipiv + r0, r0, info, c0, moves);
+    ZH_LAUNCH_CHECK();
+    return true;
+  }
+  void* ws = nullptr;
+  LeafState& st = leaf_state(s, &ws);
   const int G = (int)((M + PT - 1) / PT);
   if (G > panel::GMAX || G > st.max_resident)
     throw std::runtime_error("getrf: the matrix is too tall for one resident panel grid");
   const panel::WS w_ = panel::carve(ws);
-  if (G == 1) {
-    hipLaunchKernelGGL((panel::leaf_kernel<T, false>), dim3(1), dim3(PT), 0, s, M, w,
-                       A + r0 * lda + c0, lda, ipiv + r0, r0, info, c0, w_, 0u, 0L);
-  } else {
-    // tags of this launch: base + 1 .. base + 64, above every earlier launch's
-    const uint32_t base = (uint32_t)st.launches * (uint32_t)(panel::W + 1);
-    st.launches++;
-    if (leaf_lookahead())
-      hipLaunchKernelGGL((panel::leaf_la_kernel<T>), dim3(G), dim3(panel::la_threads<T>()), 0, s, M, w, A + r0 * lda + c0, lda,
-                         ipiv + r0, r0, info, c0, w_, base, panel_spin_limit());
-    else
-      hipLaunchKernelGGL((panel::leaf_kernel<T, true>), dim3(G), dim3(PT), 0, s, M, w,
-                         A + r0 * lda + c0, lda, ipiv + r0, r0, info, c0, w_, base, panel_spin_limit());
-  }
+  // tags of this launch: base + 1 .. base + 64, above every earlier launch's
+  const uint32_t base = (uint32_t)st.launches * (uint32_t)(panel::W + 1);
+  st.launches++;
+  if (leaf_lookahead())
+    hipLaunchKernelGGL((panel::leaf_la_kernel<T>), dim3(G), dim3(panel::la_threads<T>()), 0, s, M, w, A + r0 * lda + c0, lda,
+                       ipiv + r0, r0, info, c0, w_, base, panel_spin_limit());
+  else
+    hipLaunchKernelGGL((panel::leaf_kernel<T>), dim3(G), dim3(PT), 0, s, M, w,
+                       A + r0 * lda + c0, lda, ipiv + r0, r0, info, c0, w_, base, panel_spin_limit());
   ZH_LAUNCH_CHECK();
+  return false;
 }
-template void leaf_factor<double>(int64_t, double*, int64_t, int64_t, int64_t, int, int32_t*, int*, hipStream_t);
-template void leaf_factor<float>(int64_t, float*, int64_t, int64_t, int64_t, int, int32_t*, int*, hipStream_t);
+template bool leaf_factor<double>(int64_t, double*, int64_t, int64_t, int64_t, int, int32_t*, int*, int32_t*, hipStream_t);
+template bool leaf_factor<float>(int64_t, float*, int64_t, int64_t, int64_t, int, int32_t*, int*, int32_t*, hipStream_t);
 
 // Interchanges ipiv[k1..k2] (ascending) applied to `ncols` columns starting
 // at `a` of a row-major matrix, through the composed permutation. Each
@@ -131,10 +154,11 @@ void factor_panel(int64_t m, T* A, int64_t lda, int64_t j0, int64_t jb, int32_t*
                   const LuOps<T>& ops, hipStream_t s, int perm_slot) {
   for (int64_t k0 = j0; k0 < j0 + jb; k0 += panel::W) {
     const int kb = (int)std::min<int64_t>(panel::W, j0 + jb - k0);
-    leaf_factor<T>(m, A, lda, k0, k0, kb, ipiv, info, s);
+    int32_t* const pr = perm_pairs_buffer(perm_slot);
+    const bool composed = leaf_factor<T>(m, A, lda, k0, k0, kb, ipiv, info, pr, s);
     const int64_t rc = j0 + jb - (k0 + kb);
     if (k0 > j0 || rc > 0) {
-      const int32_t* pr = compose_perm((int)k0, (int)(k0 + kb - 1), ipiv, s, perm_slot);
+      if (!composed) compose_perm((int)k0, (int)(k0 + kb - 1), ipiv, s, perm_slot);
       apply_perm<T>(k0 - j0, A + j0, lda, pr, s);
       apply_perm<T>(rc, A + k0 + kb, lda, pr, s);
     }

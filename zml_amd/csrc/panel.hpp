@@ -187,11 +187,12 @@ __device__ __forceinline__ void update_row(T (&a)[W], T l, const T* __restrict__
 // Leaf LU: rows [0, M) x columns [0, Wn) of the row-major panel P (Wn <= 64).
 // ipiv[k] = piv_base + pivot row + 1 (1-based, global); *info gets
 // info_base + first zero pivot (1-based) when it is still 0.
-// MULTI: more than one workgroup (exchange through ws), else LDS only.
+// For more than one workgroup, which exchange through ws (panels of up to 1,024
+// rows take the one-workgroup leaf of panel_leaf1.hpp).
 // A wait that exceeds spin_limit polls (or any wait, when spin_limit < 0)
 // sets *ws.err and ends the kernel in every workgroup; the factors are then
 // invalid and the host reports the give-up.
-template <typename T, bool MULTI>
+template <typename T>
 __global__ void __launch_bounds__(pt_of<T>())
 leaf_kernel(int64_t M, int Wn, T* __restrict__ P, int64_t ld, int32_t* __restrict__ ipiv,
             int64_t piv_base, int* __restrict__ info, int64_t info_base, WS ws, uint32_t tag_base,
@@ -208,15 +209,15 @@ leaf_kernel(int64_t M, int Wn, T* __restrict__ P, int64_t ld, int32_t* __restric
   __shared__ T s_v[NW];
   __shared__ int64_t s_i[NW];
   __shared__ int64_t s_p;
-  __shared__ int s_nan, s_abort;
+  __shared__ int s_abort;
   __shared__ int32_t s_piv[W];
-  __shared__ T stage[MULTI ? NW : 1][W], stage_k[W];
+  __shared__ T stage[NW][W], stage_k[W];
   __shared__ int s_knan;
 
   T a[W];
 #pragma unroll
   for (int c = 0; c < W; ++c) a[c] = (own && c < Wn) ? P[i * ld + c] : T(0);
-  if (t == 0) { s_abort = 0; s_nan = 0; }
+  if (t == 0) s_abort = 0;
 
   int first_zero = 0;
   const T sfmin = sizeof(T) == 8 ? T(0x1p-1022) : T(0x1p-126);   // lamch('S')
@@ -238,7 +239,7 @@ leaf_kernel(int64_t M, int Wn, T* __restrict__ P, int64_t ld, int32_t* __restric
       s_v[wv] = wmax;
       s_i[wv] = wlane >= 0 ? (int64_t)g * PT + wv * 64 + wlane : INT64_MAX;
     }
-    if (MULTI) {
+    {
       // stage the wave's candidate row and row k for publishing (the barrier
       // below orders these writes before the publishing wave reads them)
       if (lane == wlane) {
@@ -257,22 +258,7 @@ leaf_kernel(int64_t M, int Wn, T* __restrict__ P, int64_t ld, int32_t* __restric
 #pragma unroll
     for (int w = 1; w < NW; ++w) amax(bv, bi, s_v[w], s_i[w]);
 
-    if (!MULTI) {
-      if (own && i == bi) {
-#pragma unroll
-        for (int c = 0; c < W; ++c) u[c] = a[c];
-        s_p = i;
-      }
-      if (own && i == k) {
-#pragma unroll
-        for (int c = 0; c < W; ++c) rk[c] = a[c];
-        s_nan = (ak != ak);
-      }
-      __syncthreads();
-      if (t == 0 && (s_nan || bi == INT64_MAX)) s_p = k;
-      if (s_nan && t < W) u[t] = rk[t];
-      __syncthreads();
-    } else {
+    {
       const int slot = k & 1;
       const uint32_t tag = tag_base + (uint32_t)k + 1u;
       uint64_t* my_rec = ws.rec + ((size_t)slot * GMAX + g) * REC;
