@@ -1,9 +1,8 @@
-"""The one-workgroup LU leaf (panels of up to 1,024 rows, groups of 8 columns,
-virtual interchanges) against the oracle bit for bit: a single leaf (n <= 64
-columns) has no matrix-core update in it, so factors, pivots and info equal zml's
+"""The LU leaf (groups of 8 columns, virtual interchanges; one workgroup up to 512
+rows, exchanging workgroups above) against the oracle bit for bit: a single leaf
+(n <= 64 columns) has no matrix-core update in it, so factors, pivots and info equal zml's
 exactly, at the edges of its row ranges and column groups, with exact ties, zero
-columns, subnormal pivots, infinities and NaN. At 1,025 rows the exchanging leaf
-takes over."""
+columns, subnormal pivots, infinities and NaN."""
 import numpy as np
 import pytest
 

@@ -12,14 +12,12 @@
 //     apply the panel's interchanges left and right of it (LASWP)
 //     U12 = L11^-1 A12 (TRSM), A22 -= L21 U12 (MFMA GEMM)
 //
-// Leaf kernel: G workgroups of 256 threads, thread = one panel row held in
-// registers (64 doubles). Per column k: workgroup argmax -> every workgroup
-// publishes (|a|, row) and its candidate row, then a flag barrier; each
-// workgroup then picks the global winner itself (largest |a|, lowest row on
-// ties: iamax.zig:32 uses a strict '>'), swaps, scales by fl(1/p) when
-// |p| >= sfmin and divides otherwise (getrf2.zig:65-87), and applies the
-// rank-1 update with separately rounded multiply and subtract (no FMA),
-// i.e. the very operation sequence of zml's unblocked closed form.
+// Leaf kernel (panel_leaf1.hpp): one row per thread in registers (64 values). Per
+// column the largest |a| over the rows not yet chosen, lowest position on ties
+// (iamax.zig:32 uses a strict '>'), multipliers scaled by fl(1/p) when
+// |p| >= sfmin and divided otherwise (getrf2.zig:65-87), updates with separately
+// rounded multiply and subtract (no FMA), i.e. the very operation sequence of zml's
+// unblocked closed form.
 #include "zmlhip_internal.hpp"
 #include "panel.hpp"
 #include "panel_fused.hpp"
@@ -60,26 +58,29 @@ static LeafState& leaf_state(hipStream_t s, void** ws_out) {
   }
   if (st.max_resident == 0) {
     int per_cu = 0;
-    int per_cu_la = 0;
+    int per_cu_g = 0;
     ZH_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu, panel::leaf_kernel<double>, panel::pt_of<double>(), 0));
     ZH_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu_la, panel::leaf_la_kernel<double>, panel::la_threads<double>(), 0));
-    st.max_resident = std::max(1, std::min(per_cu, per_cu_la)) * device_cu_count();
+        &per_cu_g, panel::leaf1_kernel<double, panel::pt_of<double>(), true>, panel::pt_of<double>(), 0));
+    st.max_resident = std::max(1, std::min(per_cu, per_cu_g)) * device_cu_count();
   }
   *ws_out = ws;
   return st;
 }
 
 // Factor one leaf (rows [r0, m), columns [c0, c0 + w)) of a row-major matrix.
-// Up to kLeaf1Rows rows go to one workgroup, which also writes the leaf's row
-// moves into `moves` (true); more are spread over workgroups that exchange every
-// pivot through memory, and the caller composes the moves from ipiv (false).
-// The line: 1,024 rows are what a workgroup's registers hold (512 threads, two
-// rows each, 32 columns at a time). At that height the one-workgroup leaf takes
-// 152 us, four exchanging workgroups 320 us (MI355X, FP64). A forced give-up of the
-// exchange (negative spin limit) takes the exchanging leaf as far as it goes.
-constexpr int64_t kLeaf1Rows = 1024;
+// Up to kLeaf1Rows rows go to one workgroup, more are spread over workgroups that
+// exchange every pivot through memory. Both also write the leaf's row moves into
+// `moves` (true); with the look-ahead switch off the exchanging leaf leaves it to the
+// caller to compose them from ipiv (false).
+// The line: a workgroup holds 512 rows of 64 FP64 values in its registers (89 us,
+// against 160 us for two exchanging workgroups). Two rows per thread above that, 32
+// columns at a time with the second half through memory, took 150 us at 1,000 rows:
+// what the exchange takes (165 us) within 10%, for as much code again. A forced
+// give-up of the exchange (negative spin limit) takes the exchanging leaf as far
+// down as it goes.
+constexpr int64_t kLeaf1Rows = 512;
 template <typename T>
 bool leaf_factor(int64_t m, T* A, int64_t lda, int64_t r0, int64_t c0, int w, int32_t* ipiv,
                  int* info, int32_t* moves, hipStream_t s) {
@@ -87,19 +88,13 @@ bool leaf_factor(int64_t m, T* A, int64_t lda, int64_t r0, int64_t c0, int w, in
   constexpr int PT = panel::pt_of<T>();
   if (M <= (panel_spin_limit() < 0 ? (int64_t)PT : kLeaf1Rows)) {
     T* const p = A + r0 * lda + c0;
-    constexpr int HW = sizeof(T) == 8 ? 32 : 64;   // columns of the two-rows-per-thread form
-    if (M <= 64)
-      hipLaunchKernelGGL((panel::leaf1_kernel<T, 64, 1, 64>), dim3(1), dim3(64), 0, s, (int)M, w, p, lda, ipiv + r0,
-                         r0, info, c0, moves);
-    else if (M <= 256)
-      hipLaunchKernelGGL((panel::leaf1_kernel<T, 256, 1, 64>), dim3(1), dim3(256), 0, s, (int)M, w, p, lda,
-                         ipiv + r0, r0, info, c0, moves);
-    else if (M <= 512)
-      hipLaunchKernelGGL((panel::leaf1_kernel<T, 512, 1, 64>), dim3(1), dim3(512), 0, s, (int)M, w, p, lda,
-                         ipiv + r0, r0, info, c0, moves);
-    else
-      hipLaunchKernelGGL((panel::leaf1_kernel<T, 512, 2, HW>), dim3(1), dim3(512), 0, s, (int)M, w, p, lda,
-                         ipiv + r0, r0, info, c0, moves);
+    auto go = [&](auto kernel, int nt) {
+      hipLaunchKernelGGL(kernel, dim3(1), dim3(nt), 0, s, M, w, p, lda, ipiv + r0, r0, info, c0, moves, panel::WS{},
+                         0u, 0L);
+    };
+    if (M <= 64) go(panel::leaf1_kernel<T, 64, false>, 64);
+    else if (M <= 256) go(panel::leaf1_kernel<T, 256, false>, 256);
+    else go(panel::leaf1_kernel<T, 512, false>, 512);
     ZH_LAUNCH_CHECK();
     return true;
   }
@@ -112,14 +107,15 @@ bool leaf_factor(int64_t m, T* A, int64_t lda, int64_t r0, int64_t c0, int w, in
   // tags of this launch: base + 1 .. base + 64, above every earlier launch's
   const uint32_t base = (uint32_t)st.launches * (uint32_t)(panel::W + 1);
   st.launches++;
-  if (leaf_lookahead())
-    hipLaunchKernelGGL((panel::leaf_la_kernel<T>), dim3(G), dim3(panel::la_threads<T>()), 0, s, M, w, A + r0 * lda + c0, lda,
-                       ipiv + r0, r0, info, c0, w_, base, panel_spin_limit());
+  const bool groups = leaf_lookahead();
+  if (groups)
+    hipLaunchKernelGGL((panel::leaf1_kernel<T, PT, true>), dim3(G), dim3(PT), 0, s, M, w,
+                       A + r0 * lda + c0, lda, ipiv + r0, r0, info, c0, moves, w_, base, panel_spin_limit());
   else
     hipLaunchKernelGGL((panel::leaf_kernel<T>), dim3(G), dim3(PT), 0, s, M, w,
                        A + r0 * lda + c0, lda, ipiv + r0, r0, info, c0, w_, base, panel_spin_limit());
   ZH_LAUNCH_CHECK();
-  return false;
+  return groups;
 }
 template bool leaf_factor<double>(int64_t, double*, int64_t, int64_t, int64_t, int, int32_t*, int*, int32_t*, hipStream_t);
 template bool leaf_factor<float>(int64_t, float*, int64_t, int64_t, int64_t, int, int32_t*, int*, int32_t*, hipStream_t);

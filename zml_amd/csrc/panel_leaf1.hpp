@@ -1,6 +1,6 @@
-// One-workgroup leaf of the LU panels: partial-pivoting LU of an M x W row-major
-// panel (W <= 64) whose rows all fit one workgroup, FP64 and FP32 (zml
-// lapack/getrf2.zig:14-210).
+// Leaf of the LU panels: partial-pivoting LU of an M x W row-major panel (W <= 64)
+// by one workgroup that holds all its rows, or by workgroups that exchange every
+// pivot, FP64 and FP32 (zml lapack/getrf2.zig:14-210).
 //
 // Rows never move while the leaf runs: each carries its LAPACK position, the
 // search takes the largest |a_ik| among the rows at positions >= k, the lowest
@@ -23,10 +23,11 @@
 // records' winner, reciprocal and update: about 900 cycles with one wave per SIMD),
 // then by the LDS reads of the group updates (4 cycles per value and wave). The
 // column-by-column leaf (64-column updates, staging, three barriers and register
-// interchanges in every column; above 256 rows an exchange between workgroups as
-// well) took 146 us at 200 rows, 320 us at 500 and at 1,000 rows; this one 71, 89
-// and 152 us (one MI355X, FP64, launch included).
+// interchanges in every column) took 146 us at 200 rows; this one 71 us, and 89 us
+// at 500 rows (one MI355X, FP64, launch included).
 #pragma once
+
+#include <type_traits>
 
 #include "panel.hpp"
 
@@ -34,6 +35,7 @@ namespace zmlhip {
 namespace panel {
 
 constexpr int GW = 8;    // columns of a group
+template <int N> using Place = std::integral_constant<int, N>;
 
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ int imax_step(int v) {
@@ -89,396 +91,368 @@ struct __attribute__((aligned(16))) Leaf1Rec {
   T val[GW];
 };
 
-// x[r][c] -= l[r][q] U[q ldu + c] for q = 0 .. NQ - 1 in order, 8 columns, separately
-// rounded: one row of U (an LDS broadcast) is read ahead of the one being used. The
-// empty asm keeps the elements in this order (reordered, the products are formed
-// ahead and spill).
-template <typename T, int R, int NQ>
-__device__ __forceinline__ void apply_rows(T (&x)[R][GW], const T (&l)[R][NQ], const T* U, int ldu) {
+// One wave: publishes this workgroup's candidate `mine` of column k, the KK-th of
+// its group (position, row and the values from column k on), and puts the best
+// over all G workgroups into *out.
+template <typename T, int KK>
+__device__ __forceinline__ void exchange(const Leaf1Rec<T>* mine, Leaf1Rec<T>* out, int k, int G, int wg, int lane,
+                                         const WS& ws, uint32_t tag_base, long spin_limit, int* s_abort) {
+  constexpr int VW = (int)sizeof(T) / 4, NV = VW * (GW - KK), XW = 2 + NV;
+  const uint32_t tag = tag_base + (uint32_t)k + 1u;
+  uint64_t* const x = ws.x + (size_t)(k & 1) * XWMAX * GMAX;
+  if (lane < XW)
+    st64(x + lane * GMAX + wg,
+         tagged(tag, reinterpret_cast<const uint32_t*>(mine)[2 + lane + (lane < 2 ? 0 : VW * KK)]));
+  if (spin_limit < 0) {   // give-up forced by the host (error-path tests)
+    if (lane == 0) { *s_abort = 1; atomicExch(ws.err, 1); }
+    return;
+  }
+  double v = -1.0;
+  int pos = INT32_MAX, row = 0;
+  uint32_t val[NV];
+#pragma unroll
+  for (int w = 0; w < NV; ++w) val[w] = 0;
+  long spins = 0;
+  for (int c0 = 0; c0 < G; c0 += 64) {
+    const uint64_t* const q = x + (c0 + lane < G ? c0 + lane : c0);
+    uint64_t d[XW];
+    while (true) {
+      bool ok = true;
+#pragma unroll
+      for (int w = 0; w < XW; ++w) d[w] = ld64(q + w * GMAX);
+#pragma unroll
+      for (int w = 0; w < XW; ++w) ok = ok && tag_of(d[w]) == tag;
+      if (__all(ok)) break;
+      if (++spins > spin_limit) {
+        if (lane == 0) { *s_abort = 1; atomicExch(ws.err, 1); }
+        return;
+      }
+    }
+    const int p = (int)payload(d[0]);
+    T a;
+    if constexpr (sizeof(T) == 8) a = val_of<T>(d[3], d[2]);
+    else a = __uint_as_float(payload(d[2]));
+    double f = fabs((double)a);
+    f = f == f ? f : (double)INFINITY;   // (a NaN is a candidate only at position k)
+    f = p == INT32_MAX ? -1.0 : f;
+    if (f > v || (f == v && p < pos)) {
+      v = f;
+      pos = p;
+      row = (int)payload(d[1]);
+#pragma unroll
+      for (int w = 0; w < NV; ++w) val[w] = payload(d[2 + w]);
+    }
+  }
+  if (lane == winner<64>(v, pos)) {
+    out->pos = pos;
+    out->row = row;
+#pragma unroll
+    for (int w = 0; w < NV; ++w) reinterpret_cast<uint32_t*>(out->val)[VW * KK + w] = val[w];
+  }
+}
+
+// x[c] -= l[q] U[q W + c] for q = 0 .. 7 in order, 8 columns, separately rounded: one
+// row of U (an LDS broadcast) is read ahead of the one being used. The empty asm
+// keeps the elements in this order (reordered, the products are formed ahead and
+// spill).
+template <typename T>
+__device__ __forceinline__ void apply_group(T (&x)[GW], const T (&l)[GW], const T* U) {
 #pragma clang fp contract(off)
-  constexpr bool kAhead = R == 1;   // (two rows per thread leave no registers for it)
   T u[GW], un[GW];
 #pragma unroll
   for (int c = 0; c < GW; ++c) un[c] = U[c];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
+  for (int q = 0; q < GW; ++q) {
 #pragma unroll
-    for (int c = 0; c < GW; ++c) u[c] = kAhead || q == 0 ? un[c] : U[q * ldu + c];
-    if (kAhead && q + 1 < NQ) {
+    for (int c = 0; c < GW; ++c) u[c] = un[c];
+    if (q + 1 < GW) {
 #pragma unroll
-      for (int c = 0; c < GW; ++c) un[c] = U[(q + 1) * ldu + c];
+      for (int c = 0; c < GW; ++c) un[c] = U[(q + 1) * W + c];
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int c = 0; c < GW; ++c) {
-        x[r][c] = x[r][c] - l[r][q] * u[c];
-        asm volatile("" : "+v"(x[r][c]));
-      }
+    for (int c = 0; c < GW; ++c) {
+      x[c] = x[c] - l[q] * u[c];
+      asm volatile("" : "+v"(x[c]));
+    }
   }
 }
 
-// NT threads, R rows per thread (row t + NT r), HW columns held in registers at a
-// time: 64, or 32 in two halves, the second updated from the first through
-// memory. moves (absolute rows): moves[0] the count, then (destination, source)
-// pairs, as apply_perm_kernel reads them.
+// NT threads, one row each, its 64 values in registers. moves (absolute rows):
+// moves[0] the count, then (destination, source) pairs, as apply_perm_kernel reads
+// them.
 // Memory is read and written eight lanes to a row (64-byte pieces) and changed to
 // one row per thread in LDS: a row per lane straight from memory touches 64 lines
-// with every instruction, which took as long as the elimination itself.
-template <typename T, int NT, int R, int HW>
+// with every instruction, which took 18,000 cycles of a leaf to load and 25,000 to
+// store, against 9,000 and 14,000.
+//
+// MULTI: G workgroups of NT rows each, all resident. A workgroup's candidate of
+// column k travels as tagged words (panel.hpp's protocol) that lie word by word
+// over the workgroups, so that one wave reads every workgroup's whole record (lane
+// = workgroup) in one poll and needs no second exchange for the winner's row; row
+// k needs none either, since rows do not move. (Words 2 KB apart: 512 bytes apart
+// the polls of 64 workgroups meet on fewer memory channels, 4,400 against 4,100
+// cycles.) After a group the pivot rows' later columns go the same way, once for 8
+// columns. Per column, 64 workgroups: exchange 1.7 us, the rest 0.9 us, 220 us a
+// leaf; exchanging in two dependent polls beside 64-column updates took 360 us.
+// A wait that exceeds spin_limit polls (or any, when it is negative) sets *ws.err
+// and ends the kernel in every workgroup; the factors are then invalid.
+template <typename T, int NT, bool MULTI>
 __global__ void __launch_bounds__(NT)
-leaf1_kernel(int M, int Wn, T* __restrict__ P, int64_t ld, int32_t* __restrict__ ipiv, int64_t row_base,
-             int* __restrict__ info, int64_t info_base, int32_t* __restrict__ moves) {
+leaf1_kernel(int64_t Mp, int Wn, T* __restrict__ Pp, int64_t ld, int32_t* __restrict__ ipiv, int64_t row_base,
+             int* __restrict__ info, int64_t info_base, int32_t* __restrict__ moves, WS ws, uint32_t tag_base,
+             long spin_limit) {
 #pragma clang fp contract(off)
-  constexpr int NW = NT / 64, NG = HW / GW, TLD = GW + 1, RPP = NT / GW;   // RPP: rows of one tile pass
+  constexpr int NW = NT / 64, NG = W / GW, TLD = GW + 1, RPP = NT / GW;   // RPP: rows of one load instruction
+  // this workgroup's rows: M rows at P, panel rows rb ..
+  const int G = MULTI ? (int)gridDim.x : 1, wg = MULTI ? (int)blockIdx.x : 0, rb = wg * NT;
+  const int M = MULTI ? (int)(Mp - rb < NT ? Mp - rb : NT) : (int)Mp;
+  T* const P = Pp + (int64_t)rb * ld;
   __shared__ Leaf1Rec<T> rec[GW][NW];
-  __shared__ __attribute__((aligned(16))) T U[GW][HW];     // the group's pivot rows, later columns
+  __shared__ Leaf1Rec<T> grec[MULTI ? GW : 1];         // the winners over all workgroups
+  __shared__ __attribute__((aligned(16))) T U[GW][W];   // the group's pivot rows
   __shared__ T tile[2][NT * TLD];
   __shared__ int32_t s_pos[NT];
-  __shared__ int s_cnt;
+  __shared__ int s_cnt, s_abort;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int tr = t / GW, tc = t % GW;   // this thread's row and column in a tile pass
+  const int tr = t / GW, tc = t % GW;   // this thread's row and column of a pass
   const T sfmin = sizeof(T) == 8 ? T(0x1p-1022) : T(0x1p-126);   // lamch('S')
-  if (t == 0) s_cnt = 0;
-  int buf = 0, fz = 0, mypos = 0, myrow = 0;
+  if (t == 0) { s_cnt = 0; s_abort = 0; }
+  int fz = 0, mypos = 0, myrow = 0, kdone = 0;
 
-  // columns [c0, c0 + 8) of rows NT r .. NT r + NT - 1, element e of this thread
-  // (row tr + RPP e), clamped into the panel; keep8 makes zeros of what lies outside.
-  // Apart, so that every load is on its way before the first is waited for.
-  auto read8 = [&](int r, int c0, T (&v)[GW]) __attribute__((always_inline)) {
-    const int row0 = NT * r + tr;
-    const T* const last = P + (int64_t)(M - 1) * ld + min(c0 + tc, Wn - 1);
-    const T* p = P + (int64_t)row0 * ld + min(c0 + tc, Wn - 1);
+  int pos = t < M ? rb + t : -1;   // this row's position in the panel; -1: no row
+  T a[W];
+  // pass g: columns [8 g, 8 g + 8) of every row, element e of this thread at row
+  // tr + RPP e; all loads are on their way before the first is waited for (clamped
+  // into the panel, then masked), and each pass changes layout in LDS
+  {
+    T v[NG][GW];
 #pragma unroll
-    for (int e = 0; e < GW; ++e) {
-      v[e] = *(row0 + RPP * e < M ? p : last);
-      p += (int64_t)RPP * ld;
-    }
-  };
-  auto keep8 = [&](int r, int c0, T (&v)[GW]) __attribute__((always_inline)) {
+    for (int g = 0; g < NG; ++g) {
+      const int64_t col = min(GW * g + tc, Wn - 1);
+      const T* const last = P + (int64_t)(M - 1) * ld + col;
+      const T* p = P + (int64_t)tr * ld + col;
 #pragma unroll
-    for (int e = 0; e < GW; ++e) {
-      asm volatile("" : "+v"(v[e]));
-      v[e] = (NT * r + tr + RPP * e < M && c0 + tc < Wn) ? v[e] : T(0);
-    }
-  };
-  // the pass's elements to one row per thread, and back
-  auto to_rows = [&](T (&v)[GW]) __attribute__((always_inline)) {
-    T* const q = tile[buf];
-#pragma unroll
-    for (int e = 0; e < GW; ++e) q[(tr + RPP * e) * TLD + tc] = v[e];
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < GW; ++c) v[c] = q[t * TLD + c];
-    buf ^= 1;
-  };
-  auto to_pass = [&](const T (&x)[GW], T (&v)[GW]) __attribute__((always_inline)) {
-    T* const q = tile[buf];
-#pragma unroll
-    for (int c = 0; c < GW; ++c) q[t * TLD + c] = x[c];
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < GW; ++e) v[e] = q[(tr + RPP * e) * TLD + tc];
-    buf ^= 1;
-  };
-  // a pass to memory: rows to `rows[]` (their final positions; s_pos) or to their own place
-  auto write8 = [&](int r, int c0, const T (&v)[GW], const int32_t* rows) __attribute__((always_inline)) {
-    const int col = c0 + tc;
-#pragma unroll
-    for (int e = 0; e < GW; ++e) {
-      const int row = NT * r + tr + RPP * e;
-      if (row < M && col < Wn) P[(int64_t)(rows ? rows[tr + RPP * e] : row) * ld + col] = v[e];
-    }
-  };
-
-  int pos[R];
-  T a[R][HW];
-  auto load_half = [&](int c0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      T v[NG][GW];
-#pragma unroll
-      for (int g = 0; g < NG; ++g) read8(r, c0 + GW * g, v[g]);
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        keep8(r, c0 + GW * g, v[g]);
-        to_rows(v[g]);
-#pragma unroll
-        for (int c = 0; c < GW; ++c) a[r][GW * g + c] = v[g][c];
+      for (int e = 0; e < GW; ++e) {
+        v[g][e] = *(tr + RPP * e < M ? p : last);
+        p += (int64_t)RPP * ld;
       }
     }
-  };
 #pragma unroll
-  for (int r = 0; r < R; ++r) pos[r] = t + NT * r < M ? t + NT * r : -1;   // -1: no row
-  load_half(0);
-
-  for (int h0 = 0; h0 < Wn; h0 += HW) {
     for (int g = 0; g < NG; ++g) {
-      const int k0 = h0 + GW * g;
-      if (k0 >= Wn) break;
-      T w[R][GW];   // the group's columns
-      int wins[GW] = {};   // the waves whose records hold the group's pivot rows
+      T* const q = tile[g & 1];
 #pragma unroll
-      for (int gg = 0; gg < NG; ++gg)
-        if (gg == g) {
+      for (int e = 0; e < GW; ++e) {
+        asm volatile("" : "+v"(v[g][e]));
+        q[(tr + RPP * e) * TLD + tc] = (tr + RPP * e < M && GW * g + tc < Wn) ? v[g][e] : T(0);
+      }
+      __syncthreads();
 #pragma unroll
-          for (int r = 0; r < R; ++r)
+      for (int c = 0; c < GW; ++c) a[GW * g + c] = q[t * TLD + c];
+    }
+  }
+
+  // gave up: the columns not reached keep their rows (identity interchanges, no moves)
+  auto give_up = [&]() __attribute__((always_inline)) {
+    if (wg == 0) {
+      if (t < Wn) ipiv[t] = (int32_t)(row_base + (t < kdone ? mypos : t) + 1);
+      if (t == 0) moves[0] = 0;
+    }
+  };
+  for (int g = 0; g < NG; ++g) {
+    const int k0 = GW * g;
+    if (k0 >= Wn) break;
+    T w[GW];   // the group's columns
 #pragma unroll
-            for (int c = 0; c < GW; ++c) w[r][c] = a[r][GW * gg + c];
-        }
+    for (int gg = 0; gg < NG; ++gg)
+      if (gg == g) {
 #pragma unroll
-      for (int kk = 0; kk < GW; ++kk) {
-        const int k = k0 + kk;
-        if (k >= Wn) break;
-        // the thread's, then the wave's candidate; a NaN at position k keeps it (as
-        // +inf at the lowest position), elsewhere a NaN never wins
-        double bv = -1.0;
-        int bp = INT32_MAX, br = 0;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          double f = fabs((double)w[r][kk]);
-          f = f == f ? f : (pos[r] == k ? (double)INFINITY : -1.0);
-          f = pos[r] >= k ? f : -1.0;
-          if (f > bv || (R > 1 && f == bv && pos[r] < bp)) { bv = f; bp = pos[r]; br = r; }
-        }
-        const int wl = winner<64>(bv, bp);
+        for (int c = 0; c < GW; ++c) w[c] = a[GW * gg + c];
+      }
+    // one column, its place in the group a constant (a loop over it is not unrolled
+    // whole at this size, and indexing registers is slow); false: gave up
+    auto column = [&](auto place) __attribute__((always_inline)) {
+      constexpr int kk = decltype(place)::value;
+      const int k = k0 + kk;
+      if (k >= Wn) return true;
+      // the wave's candidate; a NaN at position k keeps it (as +inf at the lowest
+      // position), elsewhere a NaN never wins
+      double f = fabs((double)w[kk]);
+      f = f == f ? f : (pos == k ? (double)INFINITY : -1.0);
+      f = pos >= k ? f : -1.0;
+      const int bp = f >= 0.0 ? pos : INT32_MAX;
+      if (lane == winner<64>(f, bp)) {
         Leaf1Rec<T>* const my = &rec[kk][wv];
-        if (lane == wl) {
-          my->v = bv;
-          my->pos = bp;
-          my->row = t + NT * br;
+        my->v = f;
+        my->pos = bp;
+        my->row = rb + t;
 #pragma unroll
-          for (int c = 0; c < GW; ++c) {
-            T x = w[0][c];
-#pragma unroll
-            for (int r = 1; r < R; ++r) x = br == r ? w[r][c] : x;
-            my->val[c] = x;
-          }
-        }
-        __syncthreads();
-        const Leaf1Rec<T>* const q = &rec[kk][NW > 1 ? lane % NW : 0];
-        const double qv = q->v;
-        const int qp = q->pos, qr = q->row;
-        const int ww = NW > 1 ? winner<NW == 1 ? 64 : NW>(qv, qp) : 0;
-        const int ppos = __builtin_amdgcn_readlane(qp, ww), prow = __builtin_amdgcn_readlane(qr, ww);
-        const T* const win = rec[kk][ww].val;
-        T u[GW];
-#pragma unroll
-        for (int c = kk; c < GW; ++c) u[c] = win[c];
-        const T piv = u[kk];
-        // uniform over the workgroup: a zero pivot makes no interchange (getrf2.zig:55; ppos is k
-        // then), one below sfmin divides
-        const bool nz = __builtin_amdgcn_readfirstlane(piv != T(0)) != 0;
-        const bool recip = __builtin_amdgcn_readfirstlane(fabs(piv) >= sfmin) != 0;
-        if (!nz && fz == 0) fz = k + 1;
-        mypos = lane == k ? ppos : mypos;   // lane k keeps column k's pivot
-        myrow = lane == k ? prow : myrow;
-        wins[kk] = ww;
-        T l[R];
-        if (recip) {
-          const T rinv = T(1) / piv;
-#pragma unroll
-          for (int r = 0; r < R; ++r) l[r] = w[r][kk] * rinv;
-        } else {
-#pragma unroll
-          for (int r = 0; r < R; ++r) l[r] = nz ? w[r][kk] / piv : w[r][kk];
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const bool is_piv = prow == t + NT * r;
-          if (pos[r] >= k && !is_piv) {
-            w[r][kk] = l[r];
-#pragma unroll
-            for (int c = kk + 1; c < GW; ++c) w[r][c] = w[r][c] - l[r] * u[c];
-            if (pos[r] == k) pos[r] = ppos;
-          }
-          if (is_piv) pos[r] = k;
-        }
+        for (int c = 0; c < GW; ++c) my->val[c] = w[c];
       }
+      __syncthreads();
+      const Leaf1Rec<T>* const q = &rec[kk][NW > 1 ? lane % NW : 0];
+      const double qv = q->v;
+      const int qp = q->pos, qr = q->row;
+      const int ww = NW > 1 ? winner<NW == 1 ? 64 : NW>(qv, qp) : 0;
+      int ppos, prow;
+      const T* win;
+      if constexpr (MULTI) {
+        if (wv == 0)
+          exchange<T, kk>(&rec[kk][ww], &grec[kk], k, G, wg, lane, ws, tag_base, spin_limit, &s_abort);
+        __syncthreads();
+        if (s_abort) return false;
+        ppos = grec[kk].pos;
+        prow = grec[kk].row;
+        win = grec[kk].val;
+      } else {
+        ppos = __builtin_amdgcn_readlane(qp, ww);
+        prow = __builtin_amdgcn_readlane(qr, ww);
+        win = rec[kk][ww].val;
+      }
+      T u[GW];
+#pragma unroll
+      for (int c = kk; c < GW; ++c) u[c] = win[c];
+      const T piv = u[kk];
+      // uniform over the workgroup: a zero pivot makes no interchange (getrf2.zig:55; ppos is k
+      // then), one below sfmin divides
+      const bool nz = __builtin_amdgcn_readfirstlane(piv != T(0)) != 0;
+      const bool recip = __builtin_amdgcn_readfirstlane(fabs(piv) >= sfmin) != 0;
+      if (!nz && fz == 0) fz = k + 1;
+      mypos = lane == k ? ppos : mypos;   // lane k keeps column k's pivot
+      myrow = lane == k ? prow : myrow;
+      kdone = k + 1;
+      T l = w[kk];
+      if (recip) {
+        const T rinv = T(1) / piv;
+        l = l * rinv;
+      } else if (nz) {
+        l = l / piv;
+      }
+      const bool is_piv = prow == rb + t;
+      if (pos >= k && !is_piv) {
+        w[kk] = l;
+#pragma unroll
+        for (int c = kk + 1; c < GW; ++c) w[c] = w[c] - l * u[c];
+        if (pos == k) pos = ppos;
+      }
+      if (is_piv) pos = k;
+      return true;
+    };
+    if (!(column(Place<0>{}) && column(Place<1>{}) && column(Place<2>{}) && column(Place<3>{}) &&
+          column(Place<4>{}) && column(Place<5>{}) && column(Place<6>{}) && column(Place<7>{}))) {
+      give_up();
+      return;
+    }
+#pragma unroll
+    for (int gg = 0; gg < NG; ++gg)
+      if (gg == g) {
+#pragma unroll
+        for (int c = 0; c < GW; ++c) a[GW * gg + c] = w[c];
+      }
+    if (g + 1 >= NG || k0 + GW >= Wn) continue;
+    // U of the group's rows: their later columns, u_q = a_q - sum_{j < q} l_qj u_j
+    // in order (with the group's columns, which hold the multipliers l)
+    if (pos >= k0 && pos < k0 + GW) {
 #pragma unroll
       for (int gg = 0; gg < NG; ++gg)
-        if (gg == g) {
+        if (gg >= g) {
 #pragma unroll
-          for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int c = 0; c < GW; ++c) a[r][GW * gg + c] = w[r][c];
+          for (int c = 0; c < GW; ++c) U[pos - k0][GW * gg + c] = a[GW * gg + c];
         }
-      if (g + 1 >= NG || k0 + GW >= Wn) continue;
-      // U of the group's rows: their later columns, u_q = a_q - sum_{j < q} l_qj u_j
-      // in order (a pivot row's multipliers are the first values of its record)
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (pos[r] >= k0 && pos[r] < k0 + GW) {
-#pragma unroll
-          for (int gg = 1; gg < NG; ++gg)
-            if (gg > g) {
-#pragma unroll
-              for (int c = 0; c < GW; ++c) U[pos[r] - k0][GW * gg + c] = a[r][GW * gg + c];
-            }
-        }
-      __syncthreads();
-      const int cu = GW * (g + 1) + t;
-      if (cu < HW) {
-        T x[GW];
-#pragma unroll
-        for (int q = 0; q < GW; ++q) x[q] = U[q][cu];
-#pragma unroll
-        for (int q = 1; q < GW; ++q) {
-          const T* const lq = rec[q][wins[q]].val;
-#pragma unroll
-          for (int j = 0; j < q; ++j) x[q] = x[q] - lq[j] * x[j];
-          U[q][cu] = x[q];
+    }
+    __syncthreads();
+    if constexpr (MULTI) {
+      // between the workgroups: this one's pivot rows go out, the others' come in
+      // (everything goes out before anything is waited for)
+      const int rest = W - k0;
+      const uint32_t tag = tag_base + (uint32_t)(k0 + GW);
+      uint64_t* const xu = ws.u + (size_t)(g & 1) * GW * W * 2;
+      for (int e = t; e < GW * rest; e += NT) {
+        const int q = e / rest, c = k0 + e % rest;
+        if (grec[q].row / NT == wg) st_val<T>(xu + 2 * (q * W + c), tag, U[q][c]);
+      }
+      for (int e = t; e < GW * rest; e += NT) {
+        const int q = e / rest, c = k0 + e % rest;
+        if (grec[q].row / NT == wg) continue;
+        const uint64_t* const x = xu + 2 * (q * W + c);
+        long spins = 0;
+        while (true) {
+          const uint64_t hi = ld64(x), lo = ld64(x + 1);
+          if (tag_of(hi) == tag && tag_of(lo) == tag) {
+            U[q][c] = val_of<T>(hi, lo);
+            break;
+          }
+          if (++spins > spin_limit) { s_abort = 1; atomicExch(ws.err, 1); break; }
+          __builtin_amdgcn_s_sleep(1);
         }
       }
       __syncthreads();
-#pragma unroll
-      for (int gg = 1; gg < NG; ++gg)
-        if (gg > g) {
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            if (pos[r] >= k0 + GW) {
-              T x[1][GW], l[1][GW];
-#pragma unroll
-              for (int c = 0; c < GW; ++c) { x[0][c] = a[r][GW * gg + c]; l[0][c] = w[r][c]; }
-              apply_rows<T, 1, GW>(x, l, &U[0][GW * gg], HW);
-#pragma unroll
-              for (int c = 0; c < GW; ++c) a[r][GW * gg + c] = x[0][c];
-            } else if (pos[r] >= k0) {   // pivoted in this group: its solved values
-#pragma unroll
-              for (int c = 0; c < GW; ++c) a[r][GW * gg + c] = U[pos[r] - k0][GW * gg + c];
-            }
-          }
-        }
+      if (s_abort) { give_up(); return; }
     }
-    if constexpr (HW < W) {
-      if (h0 + HW < Wn) {
-        // the second half: the pivot rows' columns (U12) by substitution, then
-        // every other row, 8 columns at a time; this half's columns to memory, in place
-        __shared__ int32_t s_prow[W];
-        __shared__ T L11[HW][HW + 1];
-        __shared__ __attribute__((aligned(16))) T U12[HW][HW];
-        const int h1 = h0 + HW;
-        if (t < W) s_prow[t] = myrow;
-        __syncthreads();
+    const int cu = k0 + GW + t;
+    if (cu < W) {
+      T x[GW];
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-          if (pos[r] >= 0 && pos[r] < h1) {
+      for (int q = 0; q < GW; ++q) x[q] = U[q][cu];
 #pragma unroll
-            for (int c = 0; c < HW; ++c) L11[pos[r]][c] = a[r][c];
-          }
-        for (int e = t; e < HW * HW; e += NT) {
-          const int q = e / HW, c = e % HW;
-          U12[q][c] = h1 + c < Wn ? P[(int64_t)s_prow[q] * ld + h1 + c] : T(0);
-        }
+      for (int q = 1; q < GW; ++q) {
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-          for (int g = 0; g < NG; ++g) {
-            T x[GW], v[GW];
-#pragma unroll
-            for (int c = 0; c < GW; ++c) x[c] = a[r][GW * g + c];
-            to_pass(x, v);
-            write8(r, h0 + GW * g, v, nullptr);
-          }
-        __syncthreads();
-        for (int b = 0; b < HW; b += GW) {
-          if (t < HW) {   // the block's 8 rows of column t, in order
-            T x[GW];
-#pragma unroll
-            for (int q = 0; q < GW; ++q) x[q] = U12[b + q][t];
-#pragma unroll
-            for (int q = 1; q < GW; ++q) {
-#pragma unroll
-              for (int j = 0; j < q; ++j) x[q] = x[q] - L11[b + q][b + j] * x[j];
-              U12[b + q][t] = x[q];
-            }
-          }
-          __syncthreads();
-          for (int e = t; e < (HW - b - GW) * HW; e += NT) {   // the rows below it
-            const int q = b + GW + e / HW, c = e % HW;
-            T x = U12[q][c];
-#pragma unroll
-            for (int j = 0; j < GW; ++j) x = x - L11[q][b + j] * U12[b + j][c];
-            U12[q][c] = x;
-          }
-          __syncthreads();
-        }
-        for (int cg = 0; cg < HW; cg += GW) {
-          T x[R][GW];
-#pragma unroll
-          for (int r = 0; r < R; ++r) read8(r, h1 + cg, x[r]);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            keep8(r, h1 + cg, x[r]);
-            to_rows(x[r]);
-          }
-          apply_rows<T, R, HW>(x, a, &U12[0][cg], HW);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            T v[GW];
-            if (pos[r] >= 0 && pos[r] < h1) {
-#pragma unroll
-              for (int c = 0; c < GW; ++c) x[r][c] = U12[pos[r]][cg + c];
-            }
-            to_pass(x[r], v);
-            write8(r, h1 + cg, v, nullptr);
-          }
-        }
-        // (written by other threads of this workgroup: through L1, in order)
-        __threadfence_block();
-        __syncthreads();
-        load_half(h1);
+        for (int j = 0; j < q; ++j) x[q] = x[q] - U[q][k0 + j] * x[j];
+        U[q][cu] = x[q];
       }
     }
+    __syncthreads();
+#pragma unroll
+    for (int gg = 1; gg < NG; ++gg)
+      if (gg > g) {
+        if (pos >= k0 + GW) {
+          T x[GW];
+#pragma unroll
+          for (int c = 0; c < GW; ++c) x[c] = a[GW * gg + c];
+          apply_group<T>(x, w, &U[0][GW * gg]);
+#pragma unroll
+          for (int c = 0; c < GW; ++c) a[GW * gg + c] = x[c];
+        } else if (pos >= k0) {   // pivoted in this group: its solved values
+#pragma unroll
+          for (int c = 0; c < GW; ++c) a[GW * gg + c] = U[pos - k0][GW * gg + c];
+        }
+      }
   }
 
-  // rows to their final positions; every row of the panel has been read
-  if constexpr (HW < W) {
-    if (Wn > HW) {
-      // the first half of the rows that move, 8 columns at a time
-      for (int c0 = 0; c0 < HW; c0 += GW) {
-        T x[R][GW];
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          if (pos[r] >= 0 && pos[r] != t + NT * r) {
-#pragma unroll
-            for (int c = 0; c < GW; ++c) x[r][c] = P[(int64_t)(t + NT * r) * ld + c0 + c];
-          }
-        __builtin_amdgcn_s_waitcnt(0xF70);   // (loads returned before any row is overwritten)
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          if (pos[r] >= 0 && pos[r] != t + NT * r) {
-#pragma unroll
-            for (int c = 0; c < GW; ++c) P[(int64_t)pos[r] * ld + c0 + c] = x[r][c];
-          }
-      }
-    }
-  }
-  const int cl = HW < W && Wn > HW ? HW : 0;   // first column still in registers
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    __syncthreads();
-    s_pos[t] = pos[r];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      T x[GW], v[GW];
-#pragma unroll
-      for (int c = 0; c < GW; ++c) x[c] = a[r][GW * g + c];
-      to_pass(x, v);
-      write8(r, cl + GW * g, v, s_pos);
-    }
-    if (pos[r] >= 0 && pos[r] != t + NT * r) {
-      const int q = atomicAdd(&s_cnt, 1);
-      moves[1 + 2 * q] = (int32_t)(row_base + pos[r]);
-      moves[2 + 2 * q] = (int32_t)(row_base + t + NT * r);
-    }
-  }
+  // rows to their final positions (every workgroup's rows were read before its
+  // first exchange), pass by pass
   __syncthreads();
-  if (t < Wn) ipiv[t] = (int32_t)(row_base + mypos + 1);
-  if (t == 0) {
-    moves[0] = s_cnt;
-    if (fz != 0 && *info == 0) *info = (int)(info_base + fz);
+  s_pos[t] = pos;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    T* const q = tile[g & 1];
+#pragma unroll
+    for (int c = 0; c < GW; ++c) q[t * TLD + c] = a[GW * g + c];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < GW; ++e) {
+      const int row = tr + RPP * e;
+      if (row < M && GW * g + tc < Wn) Pp[(int64_t)s_pos[row] * ld + GW * g + tc] = q[row * TLD + tc];
+    }
+  }
+  // the moves: every pivot row to its position, and the rows that held those
+  // positions to where the interchanges left them (all known to workgroup 0)
+  if (wg == 0) {
+    if (t < Wn && myrow != t) {
+      const int q = atomicAdd(&s_cnt, 1);
+      moves[1 + 2 * q] = (int32_t)(row_base + t);
+      moves[2 + 2 * q] = (int32_t)(row_base + myrow);
+    }
+    if (t < Wn && pos >= Wn) {
+      const int q = atomicAdd(&s_cnt, 1);
+      moves[1 + 2 * q] = (int32_t)(row_base + pos);
+      moves[2 + 2 * q] = (int32_t)(row_base + t);
+    }
+    __syncthreads();
+    if (t < Wn) ipiv[t] = (int32_t)(row_base + mypos + 1);
+    if (t == 0) {
+      moves[0] = s_cnt;
+      if (fz != 0 && *info == 0) *info = (int)(info_base + fz);
+    }
   }
 }
 
