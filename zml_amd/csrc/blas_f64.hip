@@ -168,16 +168,16 @@ inline int grid_for(int64_t n, int threads = 256, int cap = 65536) {
 // ---------------------------------------------------------------------------
 template <typename T>
 void syrk_cm(int uplo, int trans, int64_t n, int64_t k, T alpha, const T* a, int64_t lda, T beta, T* c,
-             int64_t ldc, hipStream_t s) {
+             int64_t ldc, hipStream_t s, int split_slot) {
   if (n <= 0) return;
   const int ta = is_notrans(trans) ? kNoTrans : kTrans;
   const int tb = is_notrans(trans) ? kTrans : kNoTrans;
-  gemm_cm<T>(ta, tb, n, n, k, alpha, a, lda, a, lda, beta, c, ldc, s, uplo);
+  gemm_cm<T>(ta, tb, n, n, k, alpha, a, lda, a, lda, beta, c, ldc, s, uplo, split_slot);
 }
 template void syrk_cm<double>(int, int, int64_t, int64_t, double, const double*, int64_t, double, double*,
-                              int64_t, hipStream_t);
+                              int64_t, hipStream_t, int);
 template void syrk_cm<float>(int, int, int64_t, int64_t, float, const float*, int64_t, float, float*,
-                             int64_t, hipStream_t);
+                             int64_t, hipStream_t, int);
 
 void syrk_f64_cm(int uplo, int trans, int64_t n, int64_t k, double alpha, const double* a,
                  int64_t lda, double beta, double* c, int64_t ldc, hipStream_t s) {

@@ -101,6 +101,7 @@ struct DevBuf {
 };
 
 // ---- validated device implementations (throw on HIP errors) ---------------------
+constexpr int kSplitSlot = 26;   // workspace slot of the GEMM entry points' partial sums
 
 // gemm.zig:14-65 mapping + :98-101 checks (T = double for dgemm, float for sgemm)
 template <typename T>
@@ -121,7 +122,7 @@ int gemm_dev(int layout, int transa, int transb, int m, int n, int k, T alpha, c
   if (ldb < std::max(1, nrowb)) return layout == kRowMajor ? -9 : -11;
   if (ldc < std::max(1, m)) return -14;
   if (m == 0 || n == 0 || ((alpha == T(0) || k == 0) && beta == T(1))) return 0;
-  gemm_cm<T>(transa, transb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, 0);
+  gemm_cm<T>(transa, transb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, 0, kSplitSlot);
   return 0;
 }
 
@@ -168,7 +169,7 @@ int syrk_dev(int layout, int uplo, int trans, int n, int k, T alpha, const T* a,
   if (lda < std::max(1, nrowa)) return -8;
   if (ldc < std::max(1, n)) return -11;
   if (n == 0 || ((alpha == T(0) || k == 0) && beta == T(1))) return 0;
-  syrk_cm<T>(uplo, trans, n, k, alpha, a, lda, beta, c, ldc, s);
+  syrk_cm<T>(uplo, trans, n, k, alpha, a, lda, beta, c, ldc, s, kSplitSlot);
   return 0;
 }
 

@@ -9,21 +9,25 @@
 // zml's separately rounded loop to within the usual gamma_k |A||B| bound
 // (bitwise on integer-valued data such as the reference's golden vectors).
 //
-// Tiling: a 256-thread workgroup computes a 128 x 128 tile of C; its four
-// waves each own 64 x 64 (4 x 4 MFMA tiles of 16 x 16). K advances in slabs
-// of 16 staged through double-buffered LDS (both operands stored k-major,
-// so every MFMA operand fetch is a 16-lane contiguous read). The MFMA is
-// issued as C^T = op(B)^T op(A)^T so that the 16 lanes of an output group
-// hold 16 consecutive rows of one column of C: stores and beta-loads are
-// 128-byte contiguous in column-major memory. The two element types differ
-// only in the MFMA and in which output row a lane's accumulator r holds
-// (FP64: lane / 16 + 4 r; FP32: 4 (lane / 16) + r).
-//
-// FP64 products whose shapes allow it (whole k-slabs, 16-byte aligned operand
-// columns) take a second kernel with the same tile and arithmetic whose
-// operand slabs go from global memory to LDS by the load unit
-// (gemm_dma_f64_kernel below): 53.6 -> 64.4 TF/s for the K = 512 update of a
-// 16384 x 16384 matrix, 59.5 -> 71.4 TF/s for 8192^3 on MI355X, same bits.
+// Two kernels, with the same order of operations for every element of C (the same
+// bits), chosen in gemm_cm:
+//  - gemm_dma_f64_kernel (FP64, whole k-slabs, 16-byte aligned operand columns):
+//    128 x 128 tiles whose operand slabs go from global memory to LDS by the load
+//    unit; 71 TF/s at 4096^3 and above on MI355X;
+//  - gemm_small_kernel (every shape, FP64 and FP32): 64 x 64 tiles staged through
+//    registers, four workgroups per CU, with k split over workgroups where even
+//    these are few.
+// A 256-thread workgroup's four waves each own a quarter of the tile. K advances in
+// slabs of 16 through double-buffered LDS. The MFMA is issued as C^T = op(B)^T
+// op(A)^T so that the 16 lanes of an output group hold 16 consecutive rows of one
+// column of C: stores and beta-loads are 128-byte contiguous in column-major
+// memory. The two element types differ only in the MFMA and in which output row a
+// lane's accumulator r holds (FP64: lane / 16 + 4 r; FP32: 4 (lane / 16) + r).
+// (A 128 x 128 tile staged through registers, the former kernel for everything
+// the load unit does not take, was never faster than the 64 x 64 one: 59.0 against
+// 58.3 TF/s at 4096^3 odd FP64, 99.6 against 101.6 FP32, and 13 against 28 TF/s
+// at 1000^3.)
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -79,170 +83,174 @@ __device__ __forceinline__ void tile_coords(int64_t bid, int64_t ntm, int64_t nt
   tn = r / gm;
 }
 
-template <typename T, bool TA, bool TB>
-__global__ void __launch_bounds__(NT, 2)
-gemm_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict__ A,
-            int64_t lda, const T* __restrict__ B, int64_t ldb, T beta,
-            T* __restrict__ C, int64_t ldc, int tri, int64_t tri_tiles) {
-  typedef typename Mfma<T>::acc acc_t;
-  __shared__ T As[2][BK * LDA_S];
-  __shared__ T Bs[2][BK * LDB_S];
+// ---- 64 x 64 tiles, staged through registers
+//
+// Four waves of 32 x 32, a k-slab of 16 with clamped loads whose addresses advance
+// by one addition (only the last, partial slab is masked), four workgroups per CU
+// to cover the loads: bound by LDS and load latency where the CUs are full (58 TF/s
+// FP64, 100 TF/s FP32 at 4096^3), by the number of tiles below about 2000^2.
+// Update form C <- C +- op(A) op(B) (beta 1, alpha +-1): the accumulators start
+// from C and B is staged negated for alpha -1, so the epilogue only stores.
+// part != nullptr: the K range is split over gridDim.y workgroups, each of which
+// leaves its plain sum in part + z m n (m x n, column-major) for splitk_sum_kernel.
+// On MI355X, against 128 x 128 tiles: 1001 x 1500 x 777 143 -> 78 us, 1024^3 145 ->
+// 67 us, 124 x 918 x 5130 (k split 17 ways) 838 -> 43 us.
+constexpr int SM = 64, SLD = SM + 2;
 
-  const int64_t ntm = (m + BM - 1) / BM, ntn = (n + BN - 1) / BN;
+template <typename T, bool TA, bool TB>
+__global__ void __launch_bounds__(NT, 4)
+gemm_small_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict__ A, int64_t lda,
+                  const T* __restrict__ B, int64_t ldb, T beta, T* __restrict__ C, int64_t ldc, int tri,
+                  int64_t tri_tiles, int64_t kper, T* __restrict__ part) {
+  typedef typename Mfma<T>::acc acc_t;
+  __shared__ T As[2][BK * SLD], Bs[2][BK * SLD];
+  const int64_t ntm = (m + SM - 1) / SM, ntn = (n + SM - 1) / SM;
   int64_t tm, tn;
   if (tri_tiles > 0) tri_tile_coords(blockIdx.x, tri_tiles, ntm, ntn, tri, tm, tn);
   else tile_coords(blockIdx.x, ntm, ntn, tm, tn);
-  const int64_t row0 = tm * BM, col0 = tn * BN;
-  if (tri == kLower && row0 + BM - 1 < col0) return;   // tile strictly above the diagonal
-  if (tri == kUpper && col0 + BN - 1 < row0) return;   // tile strictly below the diagonal
-
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-
-  // ---- global -> register staging (8 elements of A and 8 of B per thread)
-  T ra[8], rb[8];
-  auto load_tiles = [&](int64_t k0) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      int64_t i, l;
-      if (!TA) { i = row0 + (t & 127); l = k0 + (t >> 7) + 2 * q; }   // m-contiguous
-      else     { l = k0 + (t & 15);    i = row0 + (t >> 4) + 16 * q; } // k-contiguous
-      const bool ok = i < m && l < k;
-      ra[q] = ok ? (TA ? A[l + i * lda] : A[i + l * lda]) : T(0);
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      int64_t j, l;
-      if (TB) { j = col0 + (t & 127); l = k0 + (t >> 7) + 2 * q; }    // n-contiguous
-      else    { l = k0 + (t & 15);    j = col0 + (t >> 4) + 16 * q; }  // k-contiguous
-      const bool ok = j < n && l < k;
-      rb[q] = ok ? (TB ? B[j + l * ldb] : B[l + j * ldb]) : T(0);
-    }
-  };
-  // Update form C <- C +- op(A) op(B) (beta 1, alpha +-1): the accumulators start
-  // from C, loaded with the first operand slab, and B is staged negated for
-  // alpha -1, so the epilogue only stores.
-  const bool cinit = beta == T(1) && (alpha == T(1) || alpha == T(-1));
-  const bool negb = cinit && alpha == T(-1);
-  auto store_tiles = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      int i, l;
-      if (!TA) { i = t & 127; l = (t >> 7) + 2 * q; }
-      else     { l = t & 15;  i = (t >> 4) + 16 * q; }
-      As[buf][l * LDA_S + i] = ra[q];
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      int j, l;
-      if (TB) { j = t & 127; l = (t >> 7) + 2 * q; }
-      else    { l = t & 15;  j = (t >> 4) + 16 * q; }
-      Bs[buf][l * LDB_S + j] = negb ? -rb[q] : rb[q];
-    }
-  };
-
+  const int64_t row0 = tm * SM, col0 = tn * SM;
+  if (tri == kLower && row0 + SM - 1 < col0) return;
+  if (tri == kUpper && col0 + SM - 1 < row0) return;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave & 1, wn = wave >> 1;
   const int lr = lane & 15, lk = lane >> 4;
-  // lane holds C[i0 + lr][j0 + Mfma<T>::col(lk, r)] of each 16 x 16 tile
+  const int64_t kb = blockIdx.y * kper, ke = kb + kper < k ? kb + kper : k;
+
+  // element q of this thread: (i, l) = (t & 63, (t >> 6) + 4 q) where the operand is
+  // contiguous along m / n, ((t >> 4) + 16 q, t & 15) where it is along k
+  const T *pa[4], *pb[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int64_t ia = TA ? (t >> 4) + 16 * q : t & 63, la = TA ? t & 15 : (t >> 6) + 4 * q;
+    const int64_t jb = TB ? t & 63 : (t >> 4) + 16 * q, lb = TB ? (t >> 6) + 4 * q : t & 15;
+    const int64_t i = row0 + ia < m ? row0 + ia : m - 1, j = col0 + jb < n ? col0 + jb : n - 1;
+    pa[q] = TA ? A + (kb + la) + i * lda : A + i + (kb + la) * lda;
+    pb[q] = TB ? B + j + (kb + lb) * ldb : B + (kb + lb) + j * ldb;
+  }
+  const int64_t sa = TA ? BK : BK * lda, sb = TB ? BK * ldb : BK;   // to the next slab
+  T ra[4], rb[4];
+  auto load = [&](int64_t k0) __attribute__((always_inline)) {
+    if (k0 + BK <= ke) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        ra[q] = *pa[q];
+        rb[q] = *pb[q];
+        pa[q] += sa;
+        pb[q] += sb;
+      }
+    } else {   // the partial slab: the last column again, masked in both operands
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t la = k0 + (TA ? t & 15 : (t >> 6) + 4 * q), lb = k0 + (TB ? (t >> 6) + 4 * q : t & 15);
+        const int64_t ba = la < ke ? 0 : la - (ke - 1), bb = lb < ke ? 0 : lb - (ke - 1);
+        const T va = *(pa[q] - (TA ? ba : ba * lda)), vb = *(pb[q] - (TB ? bb * ldb : bb));
+        ra[q] = la < ke ? va : T(0);
+        rb[q] = lb < ke ? vb : T(0);
+      }
+    }
+  };
+  const bool cinit = !part && beta == T(1) && (alpha == T(1) || alpha == T(-1));
+  const bool negb = cinit && alpha == T(-1);
+  auto store = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int ia = TA ? (t >> 4) + 16 * q : t & 63, la = TA ? t & 15 : (t >> 6) + 4 * q;
+      const int jb = TB ? t & 63 : (t >> 4) + 16 * q, lb = TB ? (t >> 6) + 4 * q : t & 15;
+      As[buf][la * SLD + ia] = ra[q];
+      Bs[buf][lb * SLD + jb] = negb ? -rb[q] : rb[q];
+    }
+  };
   auto c_ok = [&](int64_t i, int64_t j) {
     return i < m && j < n && !(tri == kLower && i < j) && !(tri == kUpper && i > j);
   };
-  acc_t acc[4][4];
+  acc_t acc[2][2];
 #pragma unroll
-  for (int x = 0; x < 4; ++x)
+  for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int y = 0; y < 4; ++y) acc[x][y] = acc_t{T(0), T(0), T(0), T(0)};
-  if (cinit) {
+    for (int y = 0; y < 2; ++y)
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int64_t i = row0 + wm * 64 + 16 * x + lr;
-#pragma unroll
-      for (int y = 0; y < 4; ++y)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t j = col0 + wn * 64 + 16 * y + Mfma<T>::col(lk, r);
-          if (c_ok(i, j)) acc[x][y][r] = C[i + j * ldc];
+      for (int r = 0; r < 4; ++r) {
+        acc[x][y][r] = T(0);
+        if (cinit) {
+          const int64_t i = row0 + wm * 32 + 16 * x + lr, j = col0 + wn * 32 + 16 * y + Mfma<T>::col(lk, r);
+          const T v = C[(i < m ? i : m - 1) + (j < n ? j : n - 1) * ldc];
+          acc[x][y][r] = v;   // (outside C, or in the other triangle: computed, not stored)
         }
-    }
-  }
-
-  const int nk = (int)((k + BK - 1) / BK);
-  load_tiles(0);
-  store_tiles(0);
-  __syncthreads();
-
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) load_tiles((int64_t)(kt + 1) * BK);
-    const T* as = As[cur] + wm * 64 + lr;
-    const T* bs = Bs[cur] + wn * 64 + lr;
-#pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      const int kr = 4 * ks + lk;
-      T av[4], bv[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) av[x] = as[kr * LDA_S + 16 * x];
-#pragma unroll
-      for (int y = 0; y < 4; ++y) bv[y] = bs[kr * LDB_S + 16 * y];
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int y = 0; y < 4; ++y)
-          acc[x][y] = Mfma<T>::step(bv[y], av[x], acc[x][y]);
-    }
-    if (kt + 1 < nk) store_tiles(cur ^ 1);
+      }
+  if (kb < ke) {
+    load(kb);
+    store(0);
     __syncthreads();
+    int cur = 0;
+    for (int64_t k0 = kb; k0 < ke; k0 += BK, cur ^= 1) {
+      const bool more = k0 + BK < ke;
+      if (more) load(k0 + BK);
+      const T* as = As[cur] + wm * 32 + lr;
+      const T* bs = Bs[cur] + wn * 32 + lr;
+#pragma unroll
+      for (int ks = 0; ks < BK / 4; ++ks) {
+        const int kr = 4 * ks + lk;
+        T av[2], bv[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) av[x] = as[kr * SLD + 16 * x];
+#pragma unroll
+        for (int y = 0; y < 2; ++y) bv[y] = bs[kr * SLD + 16 * y];
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) acc[x][y] = Mfma<T>::step(bv[y], av[x], acc[x][y]);
+      }
+      if (more) store(cur ^ 1);
+      __syncthreads();
+    }
   }
-
-  // ---- epilogue
-  if (cinit) {
+  T* const out = part ? part + (int64_t)blockIdx.y * m * n : C;
+  const int64_t ldo = part ? m : ldc;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int64_t i = row0 + wm * 64 + 16 * x + lr;
+  for (int x = 0; x < 2; ++x) {
+    const int64_t i = row0 + wm * 32 + 16 * x + lr;
+    T cv[2][4];
+    const bool need_c = !part && !cinit && beta != T(0);
 #pragma unroll
-      for (int y = 0; y < 4; ++y)
+    for (int y = 0; y < 2; ++y)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t j = col0 + wn * 64 + 16 * y + Mfma<T>::col(lk, r);
-          if (c_ok(i, j)) C[i + j * ldc] = acc[x][y][r];
+      for (int r = 0; r < 4; ++r) {
+        const int64_t j = col0 + wn * 32 + 16 * y + Mfma<T>::col(lk, r);
+        cv[y][r] = (need_c && c_ok(i, j)) ? C[i + j * ldc] : T(0);
+      }
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t j = col0 + wn * 32 + 16 * y + Mfma<T>::col(lk, r);
+        if (!c_ok(i, j)) continue;
+        T v = acc[x][y][r];
+        if (!part && !cinit) {
+          v = alpha * v;
+          v = beta == T(0) ? v : (beta == T(1) ? cv[y][r] + v : beta * cv[y][r] + v);
         }
-    }
-    return;
-  }
-  // general alpha, beta: per row tile the 16 C values are all requested before any
-  // is used (one memory latency per row tile instead of one per element)
-  const bool need_c = beta != T(0);
-#pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int64_t i = row0 + wm * 64 + 16 * x + lr;
-    bool ok[4][4];
-    T cv[4][4];
-#pragma unroll
-    for (int y = 0; y < 4; ++y) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t j = col0 + wn * 64 + 16 * y + Mfma<T>::col(lk, r);
-        ok[y][r] = i < m && j < n && !(tri == kLower && i < j) && !(tri == kUpper && i > j);
-        cv[y][r] = (need_c && ok[y][r]) ? C[i + j * ldc] : T(0);
+        out[i + j * ldo] = v;
       }
-    }
-#pragma unroll
-    for (int y = 0; y < 4; ++y) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (!ok[y][r]) continue;
-        const int64_t j = col0 + wn * 64 + 16 * y + Mfma<T>::col(lk, r);
-        const T v = alpha * acc[x][y][r];
-        C[i + j * ldc] = beta == T(0) ? v : (beta == T(1) ? cv[y][r] + v : beta * cv[y][r] + v);
-      }
-    }
   }
+}
+
+// C = alpha (sum of the nz partial products, in order) + beta C
+template <typename T>
+__global__ void __launch_bounds__(256)
+splitk_sum_kernel(int64_t m, int64_t n, int nz, const T* __restrict__ part, T alpha, T beta, T* __restrict__ C,
+                  int64_t ldc, int tri) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, j = blockIdx.y;
+  if (i >= m || (tri == kLower && i < j) || (tri == kUpper && i > j)) return;
+  T s = part[i + j * m];
+  for (int z = 1; z < nz; ++z) s += part[((int64_t)z * n + j) * m + i];
+  T* const c = C + i + j * ldc;
+  const T v = alpha * s;
+  *c = beta == T(0) ? v : (beta == T(1) ? *c + v : beta * *c + v);
 }
 
 // ---- FP64 with the operand slabs moved global -> LDS by the load unit
 //
-// Same tile, waves, MFMA issue order and epilogue as gemm_kernel (its results
-// are identical bit for bit), but every thread issues 8 global_load_lds_dwordx4
+// MFMA order and epilogue as gemm_small_kernel (the results are identical bit for
+// bit) on 128 x 128 tiles (four waves of 64 x 64); every thread issues 8 global_load_lds_dwordx4
 // per 16-wide k-slab: each lane's 16 bytes land in LDS at 16 x its lane id
 // after the instruction's (wave-uniform) base, without passing through VGPRs
 // and without ds_write instructions. Two LDS buffers: slab kt + 1 is in flight
@@ -258,7 +266,7 @@ gemm_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict__ A,
 //    wave instruction moves 8 columns (lane 8 jj + s: column 8 q + jj, the pair
 //    s ^ sw).
 // For the update form with alpha = -1 the A fragments are negated after their
-// LDS reads (the register-staged kernel negates B before storing it): either
+// LDS reads (gemm_small_kernel negates B before storing it): either
 // way every product enters the accumulator as fl(c - a b).
 constexpr int DBK = 16;
 constexpr int DSLAB = DBK * LDA_S;   // doubles per operand buffer (>= 128 x 16)
@@ -484,9 +492,43 @@ void scale_cm(int64_t m, int64_t n, T beta, T* c, int64_t ldc, hipStream_t s, in
 template void scale_cm<double>(int64_t, int64_t, double, double*, int64_t, hipStream_t, int);
 template void scale_cm<float>(int64_t, int64_t, float, float*, int64_t, hipStream_t, int);
 
+// 64 x 64 tiles rather than 128 x 128 ones moved by the load unit. Both run in
+// rounds over the CUs; a CU delivers 0.27 TF/s on 128 x 128 tiles (0.24 while it has
+// only one), 0.22 on 64 x 64 ones, so a round of the first costs 3.26 (3.64) rounds
+// of the second: 2048 x 2176 x 784 (272 tiles, two rounds for one tile more than a
+// CU each) 198 against 163 us, 2048^3 (256 tiles) 277 against 322 us, 2500^2 x 2512
+// 609 against 671 us.
+static bool small_tiles(int64_t t128, int64_t t64) {
+  const int64_t cus = device_cu_count();
+  const int64_t r128 = (t128 + cus - 1) / cus, r64 = (t64 + cus - 1) / cus;
+  return (r128 == 1 ? 364 : 326 * r128) > 100 * r64;
+}
+
+template <typename T>
+static void small_gemm(bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda, const T* b,
+                       int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int64_t tiles, int64_t tri_tiles,
+                       int nz, T* part) {
+  const int64_t slabs = (k + BK - 1) / BK, kper = (slabs + nz - 1) / nz * BK;
+  const dim3 grid((unsigned)tiles, (unsigned)nz), block(NT);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles, kper,
+                       part);
+  };
+  if (!ta && !tb) go(gemm_small_kernel<T, false, false>);
+  else if (ta && !tb) go(gemm_small_kernel<T, true, false>);
+  else if (!ta && tb) go(gemm_small_kernel<T, false, true>);
+  else go(gemm_small_kernel<T, true, true>);
+  ZH_LAUNCH_CHECK();
+  if (part) {
+    hipLaunchKernelGGL(splitk_sum_kernel<T>, dim3((unsigned)((m + 255) / 256), (unsigned)n), dim3(256), 0, s, m, n, nz,
+                       (const T*)part, alpha, beta, c, ldc, tri);
+    ZH_LAUNCH_CHECK();
+  }
+}
+
 template <typename T>
 void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda,
-             const T* b, int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri) {
+             const T* b, int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int split_slot) {
   if (m <= 0 || n <= 0) return;
   if (alpha == T(0) || k <= 0) {  // gemm.zig:104-140: only the beta scaling remains
     scale_cm<T>(m, n, beta, c, ldc, s, tri);
@@ -496,9 +538,11 @@ void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, c
   const int64_t ntm = (m + BM - 1) / BM, ntn = (n + BN - 1) / BN;
   const int64_t tri_tiles = tri_tile_count(tri, ntm, ntn);
   const int64_t tiles = tri_tiles > 0 ? tri_tiles : ntm * ntn;
-  dim3 grid((unsigned)tiles), block(NT);
+  const int64_t nsm = (m + SM - 1) / SM, nsn = (n + SM - 1) / SM;
+  const int64_t stri = tri_tile_count(tri, nsm, nsn), stiles = stri > 0 ? stri : nsm * nsn;
   if constexpr (std::is_same<T, double>::value) {
-    if (gemm_dma_enabled() && dma_f64_ok(ta, tb, m, n, k, a, lda, b, ldb)) {
+    if (gemm_dma_enabled() && dma_f64_ok(ta, tb, m, n, k, a, lda, b, ldb) && !small_tiles(tiles, stiles)) {
+      const dim3 grid((unsigned)tiles), block(NT);
       if (!ta && !tb) hipLaunchKernelGGL((gemm_dma_f64_kernel<false, false>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
       else if (ta && !tb) hipLaunchKernelGGL((gemm_dma_f64_kernel<true, false>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
       else if (!ta && tb) hipLaunchKernelGGL((gemm_dma_f64_kernel<false, true>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
@@ -507,16 +551,31 @@ void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, c
       return;
     }
   }
-  if (!ta && !tb) hipLaunchKernelGGL((gemm_kernel<T, false, false>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
-  else if (ta && !tb) hipLaunchKernelGGL((gemm_kernel<T, true, false>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
-  else if (!ta && tb) hipLaunchKernelGGL((gemm_kernel<T, false, true>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
-  else hipLaunchKernelGGL((gemm_kernel<T, true, true>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
-  ZH_LAUNCH_CHECK();
+  // k is split where the tiles leave CUs idle: about two workgroups per CU, each
+  // with at least 128 of k (a split of 4 or 8 slabs no longer pays its sum)
+  int nz = 1;
+  if (split_slot >= 0 && stiles < device_cu_count())
+    nz = (int)std::max<int64_t>(1, std::min<int64_t>({2 * device_cu_count() / stiles, k / 128, 32}));
+  T* part = nullptr;
+  if (nz > 1) {
+    // the partial sums (at most 2 x CUs tiles) need a workspace: without one (no
+    // memory, or a stream under capture, where nothing may be allocated) no split
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+      try {
+        part = static_cast<T*>(workspace(sizeof(T) * (size_t)nz * m * n, split_slot));
+      } catch (const HipError&) {
+        (void)hipGetLastError();
+      }
+    }
+    if (!part) nz = 1;
+  }
+  small_gemm<T>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, stiles, stri, nz, part);
 }
 template void gemm_cm<double>(int, int, int64_t, int64_t, int64_t, double, const double*, int64_t, const double*,
-                              int64_t, double, double*, int64_t, hipStream_t, int);
+                              int64_t, double, double*, int64_t, hipStream_t, int, int);
 template void gemm_cm<float>(int, int, int64_t, int64_t, int64_t, float, const float*, int64_t, const float*,
-                             int64_t, float, float*, int64_t, hipStream_t, int);
+                             int64_t, float, float*, int64_t, hipStream_t, int, int);
 
 void scale_f64_cm(int64_t m, int64_t n, double beta, double* c, int64_t ldc, hipStream_t s, int tri) {
   scale_cm<double>(m, n, beta, c, ldc, s, tri);

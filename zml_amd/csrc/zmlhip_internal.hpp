@@ -141,10 +141,12 @@ inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 // ---- kernels exposed between translation units -----------------------------
 
 // Element-type generic forms (T = double or float) of the column-major
-// kernels below; the _f64 names are their FP64 instances.
+// kernels below; the _f64 names are their FP64 instances. split_slot >= 0 allows
+// gemm_cm to split a long k of a small product over workgroups, with the partial
+// sums in that workspace slot (entry points only: a slot serves one stream).
 template <typename T>
 void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda,
-             const T* b, int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri);
+             const T* b, int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int split_slot = -1);
 template <typename T>
 void scale_cm(int64_t m, int64_t n, T beta, T* c, int64_t ldc, hipStream_t s, int tri);
 template <typename T>
@@ -152,7 +154,7 @@ void trsm_cm(int side, int uplo, int transa, int diag, int64_t m, int64_t n, T a
              int64_t lda, T* b, int64_t ldb, hipStream_t s);
 template <typename T>
 void syrk_cm(int uplo, int trans, int64_t n, int64_t k, T alpha, const T* a, int64_t lda, T beta, T* c,
-             int64_t ldc, hipStream_t s);
+             int64_t ldc, hipStream_t s, int split_slot = -1);
 template <typename T>
 void potrf_cm(int uplo, int64_t n, T* a, int64_t lda, int* info, hipStream_t s);
 
