@@ -2073,7 +2073,9 @@ int dgesv_mixed(int layout, int64_t n, int64_t nrhs, const double* A, int64_t ld
   S.r = reinterpret_cast<double*>(small); small += sizeof(double) * n;
   S.c = reinterpret_cast<double*>(small); small += sizeof(double) * n;
   S.rowsum = reinterpret_cast<double*>(small); small += sizeof(double) * n;
-  S.z = reinterpret_cast<float*>(small); small += sizeof(float) * (n + NB_MIX);
+  // an even count: the exchange words after z have to be 8-byte aligned, or their
+  // 64-bit stores and loads are no single accesses and a tag can arrive before its value
+  S.z = reinterpret_cast<float*>(small); small += sizeof(float) * (n + (n & 1) + NB_MIX);
   S.xch = reinterpret_cast<uint64_t*>(small); small += sizeof(uint64_t) * (n + NB_MIX);
   S.serr = reinterpret_cast<int*>(small); small += 64;
   S.part = reinterpret_cast<double*>(small);
