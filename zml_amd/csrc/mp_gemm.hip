@@ -16,6 +16,8 @@
 // LDS. Lane l of a 32 x 32 block holds column l % 32 and rows
 // 8 (r / 4) + 4 ((l / 32) % 2) + r % 4 of register r, so every C access is
 // 32 consecutive floats.
+#include <algorithm>
+
 #include "zmlhip_internal.hpp"
 #include "tiles.hpp"
 #include "mixed.hpp"
@@ -242,74 +244,74 @@ mp_gemm_h_kernel(int64_t m, int64_t n, int64_t K, float alpha, const H* __restri
 }
 
 // Same product with the operand slabs streamed straight into LDS
-// (global_load_lds_dwordx4: a wave writes 1 KB, 16 rows of 64 bytes, lane l
-// the 16 bytes at 16 l) through a ring of S stages: slab kt + S - 1 is
-// requested while slab kt is multiplied, one barrier per slab and no
-// registers for staging. Within a row the four 16-byte k-chunks are stored
-// XOR-swizzled by (row >> 1) & 3 (each lane picks the global chunk that lands
-// at its position), so the MFMA operand reads of 8 consecutive rows hit
-// distinct banks. Needs K % 32 == 0 and 16-byte aligned rows; rows beyond m
-// (columns beyond n) read the last valid row, whose products land only in C
-// entries that are not stored. Operands and products are those of
-// mp_gemm_h_kernel, in the same order.
-// Defaults of the streamed kernel: ring stages, workgroups per CU the
-// register budget is fitted to, and whether C is requested before the K loop
-// or after it. Alone (m = n = 32256 and 16384, K = 512, FP16), three stages,
-// three workgroups per CU and C read after the products move 3.03 and 3.11
-// TB/s against 2.84 and 2.92 TB/s for four stages, two workgroups and C first;
-// but inside the mixed LU the third workgroup per CU takes the slots the panel
-// stream's kernels need, and the solve slows from 138 to 153 ms at n = 32768.
-// Four workgroups per CU (two stages) fall to 1.6 TB/s.
-constexpr int DL_STAGES = 4, DL_OCC = 2;
-constexpr bool DL_PREFETCH_C = true;
-__device__ __forceinline__ int dl_swz(int r) { return (r >> 1) & 3; }
+// (global_load_lds_dwordx4: a wave writes 1 KB, 8 rows of 128 bytes, lane l
+// the 16 bytes at 16 l) through two stages: slab kt + 1 is requested while
+// slab kt is multiplied, one barrier per slab and no registers for staging.
+// A slab is 64 halfs wide, so every request takes whole 128-byte cache lines:
+// the same loop with 32-wide slabs fetches each line twice and runs 9 % longer.
+// Within a row the eight 16-byte k-chunks are stored XOR-swizzled by row & 7
+// (each lane picks the global chunk that lands at its position), so the MFMA
+// operand reads of 8 consecutive rows hit distinct banks. Needs K % 64 == 0
+// and 16-byte aligned rows; rows beyond m (columns beyond n) read the last
+// valid row, whose products land only in C entries that are not stored.
+// Operands and products are those of mp_gemm_h_kernel, in the same order.
+//
+// The C traffic bounds the kernel (K = 512: 8 m n bytes of C against 2 m n K
+// operations). C is read after the products, 32 rows of a wave's tile at a
+// time, through 32-bit offsets: 149 registers; C requested before the products
+// took 190 and made the first slab wait for all of it (requests return in
+// order), and 64-bit addresses took 244 and spread the requests. NT reads and
+// stores C past the caches, which then keep the operands. Measured alone, FP16
+// operands of random values, K = 512: m = n = 29696 2563 us before, 2104 us,
+// 1794 us with NT (3.9 TB/s of C; the products without C take 1104 us); 6144,
+// whose C stays in the 256 MB last-level cache between the updates, 88, 72 and
+// 90 us. The mixed LU at n = 32768 goes from 127 to 114 ms with it.
+constexpr int DL_BK = 64;                  // halfs per slab row
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  // s_waitcnt vmcnt(N), the other counters unconstrained (gfx9 encoding)
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
-template <typename H, int S = DL_STAGES, int OCC = DL_OCC, bool PFC = DL_PREFETCH_C>
-__global__ void __launch_bounds__(NTH, OCC)
+template <typename H, bool NT>
+__global__ void __launch_bounds__(NTH, 2)
 mp_gemm_h_dl_kernel(int64_t m, int64_t n, int64_t K, float alpha, const H* __restrict__ A, int64_t lda,
                     const H* __restrict__ BT, int64_t ldb, float beta, const float* __restrict__ rs,
                     const float* __restrict__ cs, float* __restrict__ C, int64_t ldc, int lower,
                     int64_t tri_tiles) {
   typedef typename MfmaH<H>::vec V;
-  constexpr int ROWB = 64;                 // bytes per LDS row: 32 halfs
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[S][2][MT * ROWB];
+  constexpr int ROWB = 2 * DL_BK;          // bytes per LDS row
+  constexpr int IN = MT / 32;              // instructions per wave, operand and slab: 8 rows each
+  static_assert(MT == NTL && MT == 128, "32 rows of each operand per wave");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2][2][MT * ROWB];
   const int64_t ntm = (m + MT - 1) / MT, ntn = (n + NTL - 1) / NTL;
   int64_t tm, tn;
   if (tri_tiles > 0) tri_tile_coords(blockIdx.x, tri_tiles, ntm, ntn, kLower, tm, tn);
   else tile_of(blockIdx.x, ntm, ntn, tm, tn);
-  const int64_t row0 = tm * MT, col0 = tn * NTL;
+  // (in scalar registers, so that every address below is a scalar base and a lane offset)
+  const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane((int)tm) * MT;
+  const int64_t col0 = (int64_t)__builtin_amdgcn_readfirstlane((int)tn) * NTL;
   if (lower && col0 > row0 + MT - 1) return;   // tile strictly above the diagonal
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = wave & 1, wn = wave >> 1;
 
-  // wave w requests rows 32 w .. 32 w + 31 of both operands, two 16-row instructions each
-  const H* ga[2];
-  const H* gb[2];
+  // wave w requests rows 32 w .. 32 w + 31 of both operands; offsets from the tile's first row
+  const H* Ab = A + row0 * lda;
+  const H* Bb = BT + col0 * ldb;
+  uint32_t oa[IN], ob[IN];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = 32 * wave + 16 * j + (lane >> 2);
-    const int c = (lane & 3) ^ dl_swz(r);
-    const int64_t ia = row0 + r < m ? row0 + r : m - 1;
-    const int64_t jb = col0 + r < n ? col0 + r : n - 1;
-    ga[j] = A + ia * lda + 8 * c;
-    gb[j] = BT + jb * ldb + 8 * c;
+  for (int j = 0; j < IN; ++j) {
+    const int r = 32 * wave + 8 * j + (lane >> 3);
+    const int c = (lane & 7) ^ (r & 7);
+    oa[j] = (uint32_t)(min((int64_t)r, m - 1 - row0) * lda) + 8 * c;
+    ob[j] = (uint32_t)(min((int64_t)r, n - 1 - col0) * ldb) + 8 * c;
   }
-  auto issue = [&](int kt, int st) {
-    const int64_t ko = (int64_t)kt * BKH;
+  auto issue = [&](int kt) {
+    const int64_t ko = (int64_t)kt * DL_BK;
+    const int st = kt & 1;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      __builtin_amdgcn_global_load_lds((const void*)(ga[j] + ko),
-                                       (__attribute__((address_space(3))) void*)&lds[st][0][(32 * wave + 16 * j) * ROWB],
+    for (int j = 0; j < IN; ++j) {
+      __builtin_amdgcn_global_load_lds((const void*)(Ab + ko + oa[j]),
+                                       (__attribute__((address_space(3))) void*)&lds[st][0][(32 * wave + 8 * j) * ROWB],
                                        16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const void*)(gb[j] + ko),
-                                       (__attribute__((address_space(3))) void*)&lds[st][1][(32 * wave + 16 * j) * ROWB],
+      __builtin_amdgcn_global_load_lds((const void*)(Bb + ko + ob[j]),
+                                       (__attribute__((address_space(3))) void*)&lds[st][1][(32 * wave + 8 * j) * ROWB],
                                        16, 0, 0);
     }
   };
@@ -321,36 +323,31 @@ mp_gemm_h_dl_kernel(int64_t m, int64_t n, int64_t K, float alpha, const H* __res
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
-  f16v cv[2][2];
-  if (PFC) load_c(cv, m, n, beta, C, ldc, row0 + wm * 64, col0 + wn * 64, lane);
 
-  const int nk = (int)(K / BKH);
-#pragma unroll
-  for (int s0 = 0; s0 < S - 1; ++s0)
-    if (s0 < nk) issue(s0, s0);
+  const int nk = (int)(K / DL_BK);
+  issue(0);
   const int li = lane & 31, hk = lane >> 5;
   for (int kt = 0; kt < nk; ++kt) {
-    // this wave's part of slab kt has landed once at most the later slabs' requests are pending
-    if (kt + S - 2 < nk) wait_vm<4 * (S - 2)>();
-    else wait_vm<0>();
-    // every wave's part of slab kt is in LDS and stage (kt - 1) % S is no longer read:
-    // a bare barrier (the fence of __syncthreads would wait for every request in flight)
+    // this wave's part of slab kt, its only requests in flight, has landed, and
+    // its reads of the other stage are done (vmcnt(0) lgkmcnt(0))
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    // so every wave's part of slab kt is in LDS and the other stage is free
     asm volatile("s_barrier" ::: "memory");
-    if (kt + S - 1 < nk) issue(kt + S - 1, (kt + S - 1) % S);
-    const int st = kt % S;
+    if (kt + 1 < nk) issue(kt + 1);
+    const int st = kt & 1;
 #pragma unroll
-    for (int ks = 0; ks < BKH / 16; ++ks) {
+    for (int ks = 0; ks < DL_BK / 16; ++ks) {
       const int c = 2 * ks + hk;   // logical 16-byte chunk of the MFMA operand
       V av[2], bv[2];
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
         const int r = wm * 64 + 32 * x + li;
-        av[x] = *reinterpret_cast<const V*>(&lds[st][0][r * ROWB + 16 * (c ^ dl_swz(r))]);
+        av[x] = *reinterpret_cast<const V*>(&lds[st][0][r * ROWB + 16 * (c ^ (r & 7))]);
       }
 #pragma unroll
       for (int y = 0; y < 2; ++y) {
         const int r = wn * 64 + 32 * y + li;
-        bv[y] = *reinterpret_cast<const V*>(&lds[st][1][r * ROWB + 16 * (c ^ dl_swz(r))]);
+        bv[y] = *reinterpret_cast<const V*>(&lds[st][1][r * ROWB + 16 * (c ^ (r & 7))]);
       }
 #pragma unroll
       for (int x = 0; x < 2; ++x)
@@ -358,8 +355,52 @@ mp_gemm_h_dl_kernel(int64_t m, int64_t n, int64_t K, float alpha, const H* __res
         for (int y = 0; y < 2; ++y) acc[x][y] = MfmaH<H>::mma(av[x], bv[y], acc[x][y]);
     }
   }
-  if (!PFC) load_c(cv, m, n, beta, C, ldc, row0 + wm * 64, col0 + wn * 64, lane);
-  epilogue(acc, cv, m, n, alpha, beta, rs, cs, C, ldc, row0 + wm * 64, col0 + wn * 64, lane);
+
+  // C through a buffer descriptor of this wave's rows: entries of rows beyond m
+  // lie past its end, those of columns beyond n are sent there, and the buffer
+  // unit drops their accesses
+  const int64_t r0 = row0 + wm * 64, c0 = col0 + wn * 64;
+  const int64_t rv = min(m - r0, (int64_t)64);   // valid rows (columns past the 64th are another wave's)
+  constexpr int kFlags = 0x00027000, kAux = NT ? 2 : 0;   // raw 32-bit data; aux bit 1: non-temporal
+  const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(C + r0 * ldc + c0), 0, rv > 0 ? (int)(((rv - 1) * ldc + 64) * 4) : 0, kFlags);
+  const int ld4 = (int)ldc * 4;
+  int co[2];   // element r of block (bi, bj): row 32 bi + 8 (r / 4) + 4 hk + r % 4
+  float sc[2];
+#pragma unroll
+  for (int bj = 0; bj < 2; ++bj) {
+    const int64_t c = c0 + 32 * bj + li;
+    co[bj] = c < n ? 4 * hk * ld4 + 4 * (32 * bj + li) : (int)0x40000000;
+    sc[bj] = cs[min(c, n - 1)];
+  }
+#pragma unroll
+  for (int bi = 0; bi < 2; ++bi) {
+    float cv[2][16];
+#pragma unroll
+    for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        cv[bj][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                        cr, co[bj] + (32 * bi + 8 * (r >> 2) + (r & 3)) * ld4, 0, kAux));
+    __builtin_amdgcn_sched_barrier(0);   // (the scales' products would wait for their loads before the rest of C is requested)
+    f4u sr[4];
+    if (rv == 64) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sr[q] = *reinterpret_cast<const f4u*>(rs + r0 + 32 * bi + 8 * q + 4 * hk);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        sr[r >> 2][r & 3] = rs[min(r0 + 32 * bi + 8 * (r >> 2) + 4 * hk + (r & 3), m - 1)];
+    }
+#pragma unroll
+    for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float v = beta * cv[bj][r] + (alpha * sc[bj] * sr[r >> 2][r & 3]) * acc[bi][bj][r];
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), cr,
+                                              co[bj] + (32 * bi + 8 * (r >> 2) + (r & 3)) * ld4, 0, kAux);
+      }
+  }
 }
 
 // ---- FP32 ------------------------------------------------------------------------
@@ -500,10 +541,29 @@ bool f32_vec_ok(const float* A, int64_t lda, const float* B, int64_t ldb, int64_
          (reinterpret_cast<uintptr_t>(B) & 15) == 0;
 }
 
-// the streamed variant applies: whole 32-wide k-slabs, 16-byte aligned rows
-bool dl_ok(int64_t K, const void* A, int64_t lda, const void* BT, int64_t ldb) {
-  return K >= BKH && K % BKH == 0 && lda % 8 == 0 && ldb % 8 == 0 &&
-         (reinterpret_cast<uintptr_t>(A) & 15) == 0 && (reinterpret_cast<uintptr_t>(BT) & 15) == 0;
+// the streamed variant applies: an update of C with both scales, whole 64-wide
+// k-slabs, 16-byte aligned rows,
+// a tile's operands within 32-bit offsets and 64 rows of C within 2^30 bytes
+bool dl_ok(int64_t K, const void* A, int64_t lda, const void* BT, int64_t ldb, float beta, const float* rs,
+           const float* cs, int64_t ldc) {
+  return beta != 0.0f && rs && cs && K >= DL_BK && K % DL_BK == 0 && lda % 8 == 0 && ldb % 8 == 0 &&
+         (reinterpret_cast<uintptr_t>(A) & 15) == 0 && (reinterpret_cast<uintptr_t>(BT) & 15) == 0 &&
+         std::max(lda, ldb) < (int64_t(1) << 24) && ldc >= 64 && ldc < (int64_t(1) << 21);
+}
+
+// C goes past the caches once an update's C no longer fits the 256 MB
+// last-level cache, where the next update would find it (K = 512, both ways:
+// 72 us cached against 90 us at 144 MB, 2104 against 1794 us at 3.3 GB)
+template <typename H>
+void launch_h_dl(int64_t tiles, int64_t m, int64_t n, int64_t K, float alpha, const H* A, int64_t lda, const H* BT,
+                 int64_t ldb, float beta, const float* rs, const float* cs, float* C, int64_t ldc, int lower,
+                 int64_t tri_tiles, hipStream_t s) {
+  if (tiles * (MT * NTL * 4) > (int64_t(256) << 20))
+    hipLaunchKernelGGL((mp_gemm_h_dl_kernel<H, true>), dim3((unsigned)tiles), dim3(NTH), 0, s, m, n, K, alpha, A, lda,
+                       BT, ldb, beta, rs, cs, C, ldc, lower, tri_tiles);
+  else
+    hipLaunchKernelGGL((mp_gemm_h_dl_kernel<H, false>), dim3((unsigned)tiles), dim3(NTH), 0, s, m, n, K, alpha, A,
+                       lda, BT, ldb, beta, rs, cs, C, ldc, lower, tri_tiles);
 }
 
 }  // namespace
@@ -515,9 +575,8 @@ void mp_gemm_f16(int64_t m, int64_t n, int64_t K, float alpha, const _Float16* A
   const int64_t ntm = (m + MT - 1) / MT, ntn = (n + NTL - 1) / NTL;
   const int64_t tri_tiles = lower ? tri_tile_count(kLower, ntm, ntn) : 0;
   const int64_t tiles = tri_tiles > 0 ? tri_tiles : ntm * ntn;
-  if (dl_ok(K, A, lda, BT, ldb))
-    hipLaunchKernelGGL((mp_gemm_h_dl_kernel<_Float16>), dim3((unsigned)tiles), dim3(NTH), 0, s, m, n, K, alpha,
-                       A, lda, BT, ldb, beta, rs, cs, C, ldc, lower, tri_tiles);
+  if (dl_ok(K, A, lda, BT, ldb, beta, rs, cs, ldc))
+    launch_h_dl<_Float16>(tiles, m, n, K, alpha, A, lda, BT, ldb, beta, rs, cs, C, ldc, lower, tri_tiles, s);
   else
     hipLaunchKernelGGL((mp_gemm_h_kernel<_Float16>), dim3((unsigned)tiles), dim3(NTH), 0, s, m, n, K, alpha,
                        A, lda, BT, ldb, beta, rs, cs, C, ldc, lower, tri_tiles);
@@ -531,9 +590,8 @@ void mp_gemm_bf16(int64_t m, int64_t n, int64_t K, float alpha, const __bf16* A,
   const int64_t ntm = (m + MT - 1) / MT, ntn = (n + NTL - 1) / NTL;
   const int64_t tri_tiles = lower ? tri_tile_count(kLower, ntm, ntn) : 0;
   const int64_t tiles = tri_tiles > 0 ? tri_tiles : ntm * ntn;
-  if (dl_ok(K, A, lda, BT, ldb))
-    hipLaunchKernelGGL((mp_gemm_h_dl_kernel<__bf16>), dim3((unsigned)tiles), dim3(NTH), 0, s, m, n, K, alpha,
-                       A, lda, BT, ldb, beta, rs, cs, C, ldc, lower, tri_tiles);
+  if (dl_ok(K, A, lda, BT, ldb, beta, rs, cs, ldc))
+    launch_h_dl<__bf16>(tiles, m, n, K, alpha, A, lda, BT, ldb, beta, rs, cs, C, ldc, lower, tri_tiles, s);
   else
     hipLaunchKernelGGL((mp_gemm_h_kernel<__bf16>), dim3((unsigned)tiles), dim3(NTH), 0, s, m, n, K, alpha,
                        A, lda, BT, ldb, beta, rs, cs, C, ldc, lower, tri_tiles);
