@@ -266,7 +266,6 @@ __global__ void transpose_f32_kernel(int64_t kb, const float* __restrict__ src, 
 // getrf2.zig:65-87). A zero or NaN pivot sets *fail (which the block column's
 // first block, bappend == 0, overwrites: 1 or 0).
 constexpr int DB = 256;
-constexpr int DIAG_TY = 32;   // thread rows of the diagonal-block LU
 
 __device__ __forceinline__ int key_row(uint64_t k) {
   const uint32_t lo = (uint32_t)k;
@@ -292,279 +291,321 @@ __device__ __forceinline__ int wave64_max(int f) {
   return __builtin_amdgcn_readlane(f, 63);
 }
 
-// The block is eliminated in chunks of 16 columns (half a column group). One
-// wave, four block rows per lane, runs a chunk's 16 pivot steps in its
-// registers: each row's rank, the wave maximum through DPP, the pivot row
-// passed from the winning lane through LDS, the multipliers and the update of
-// the chunk's later columns, with no barrier between steps (the wave's own
-// 64 entries wait in LDS meanwhile). Then the chunk is applied to the later columns, step by
-// step: the pivot rows' values there (U12) come from a forward substitution
-// with the chunk's unit lower factor (one column per thread), and row i
-// receives a[i][c] -= l_ik u_k[c] for k in step order while it has not been
-// chosen (multiplier 0 afterwards). Every entry sees the same operations in
-// the same order as in a column-by-column elimination, so the bits are the
-// same.
-template <int TY>
-__global__ void __launch_bounds__(TY * 32) diag_getf2_kernel(float* __restrict__ P, int64_t ld,
-                                                            int32_t* __restrict__ ipiv, int base,
-                                                            int* __restrict__ fail, int32_t* __restrict__ pairs,
-                                                            int32_t* __restrict__ bpairs, int bappend) {
-  constexpr int TX = 32, RI = DB / TY, RJ = DB / TX, NT = TY * TX;
-  constexpr int CW = 16;        // chunk width: half a column group
+// The block is eliminated in chunks of 16 columns. Eight waves hold it as FP32
+// MFMA accumulators (the w-th rows 32 w .. 32 w + 31 in eight 32 x 32 tiles);
+// another, four block rows per lane, runs a chunk's 16 pivot steps in its
+// registers: each row's rank, the wave maximum through DPP, the pivot row read
+// from the winning lane into scalar registers, the multipliers and the update of
+// the chunk's later columns, with no barrier and no LDS between steps. The pivot
+// rows' values in the later columns (U12) then come from a forward substitution
+// with the chunk's unit lower factor, one column per thread, which writes them to
+// their final place; a row's later columns in the accumulators mean nothing once
+// it is chosen. The other rows subtract L21 U12 on the matrix cores: first the tile
+// with the next chunk's columns, which go to the pivoting wave, the rest while that
+// wave runs its steps. Every entry sees the same operations in the same order as
+// in a column-by-column elimination.
+// Bound by the pivoting wave's chain: of about 22,000 cycles a chunk its steps
+// take 15,700 (980 a column: rank, DPP maximum, row to scalar registers,
+// reciprocal, update), U12 and the barriers around it 3,000, the tile with the
+// next chunk 3,300. 164 us a block (one MI355X, launch included); one of sixteen
+// waves running the steps through LDS, with the others idle meanwhile and 16 x 8
+// x 8 multiply-adds a thread after every chunk, took 302 us. The bits are the same.
+constexpr int DIAG_NT = 768;   // eight waves that hold the block, one that pivots, and it with three more for U12
+__global__ void __launch_bounds__(DIAG_NT) diag_getf2_kernel(float* __restrict__ P, int64_t ld,
+                                                             int32_t* __restrict__ ipiv, int base,
+                                                             int* __restrict__ fail, int32_t* __restrict__ pairs,
+                                                             int32_t* __restrict__ bpairs, int bappend) {
+  typedef float f32x16 __attribute__((ext_vector_type(16)));
+  constexpr int CW = 16;        // chunk width: half a tile
   constexpr int CS = CW + 4;    // chunk row stride in floats (rows stay 16-byte aligned)
   constexpr int NC = DB / CW;   // chunks
-  constexpr int RL = DB / 64;   // block rows per lane of the panel wave: lane + 64 m
-  static_assert(TY == 32 && NT == 1024 && TX == 2 * CW, "32 x 32 threads, 8 x 8 entries each");
-  __shared__ __align__(16) float chunk[DB * CS];
-  __shared__ __align__(16) float lz[DB * CS];   // the multiplier each row took at each step (0 once chosen)
+  constexpr int NJ = DB / 32;   // tiles of a wave
+  constexpr int RL = DB / 64;   // block rows per lane of the pivoting wave: lane + 64 m
+  __shared__ __align__(16) float chunk[2][DB * CS];
   __shared__ __align__(16) float ubuf[CW * DB];   // row s: the chunk's pivot s on the later columns
-  __shared__ float park[64 * RI * RJ];   // the panel wave's own entries during the steps
-  __shared__ __align__(16) float prbuf[RL * CW];   // the winning lane's rows at a step
-  __shared__ int prow[DB], rstep[DB], invp[DB];   // rstep[r]: the step that chose row r, or -1
+  __shared__ __align__(16) int rstep[DB];         // the step that chose a row, or -1
+  __shared__ int prow[DB], invp[DB];
   __shared__ int nmove[DB / 64], bfirst;
   __shared__ int bad;
-  const int t = threadIdx.x, tx = t % TX, ty = t / TX, lane = t & 63, wv = t >> 6;
-  float a[RI][RJ];
-#pragma unroll
-  for (int i = 0; i < RI; ++i)
-#pragma unroll
-    for (int j = 0; j < RJ; ++j) a[i][j] = P[(int64_t)(ty + TY * i) * ld + tx + TX * j];
+  const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6);
+  // waves go to the four SIMDs in turn: the pivoting wave 0 shares its SIMD with
+  // two that are idle during its steps (with the block's waves there the steps
+  // take a third longer); waves 0, 4, 8 and 11 are the helpers 0 .. 3
+  const bool holds = wid % 4 != 0 && wid != 11;
+  const int wv = holds ? wid - wid / 4 - 1 : (wid == 11 ? 3 : wid / 4);
+  const int li = lane & 31, hk = lane >> 5;
+  const int row0 = 32 * wv + 4 * hk;   // element r of a tile: row row0 + 8 (r / 4) + r % 4, column li
   if (t < DB) rstep[t] = -1;
   if (t == 0) bad = 0;
-#pragma unroll 1
-  for (int ch = 0; ch < NC; ++ch) {
-    const int k0 = CW * ch, jg = ch >> 1, h = ch & 1;
-    const bool mine = (tx / CW) == h;   // this thread holds chunk columns (register group jg)
-    const int cx = tx % CW;
-    if (mine) {
-#pragma unroll
-      for (int j = 0; j < RJ; ++j)
-        if (j == jg) {
-#pragma unroll
-          for (int i = 0; i < RI; ++i) chunk[(ty + TY * i) * CS + cx] = a[i][j];
-        }
-    }
+  // Two paths with the same barriers, so that the pivoting wave carries none of
+  // the accumulators.
+  if (!holds) {
+    const int u = 64 * wv + lane;   // 256 threads
     __syncthreads();
-    if (wv == 0) {
-      // ---- the chunk's pivot steps
-#pragma unroll
-      for (int i = 0; i < RI; ++i)
-#pragma unroll
-        for (int j = 0; j < RJ; ++j) park[(i * RJ + j) * 64 + lane] = a[i][j];
-      float x[RL][CW];
-      bool rd[RL];
-#pragma unroll
-      for (int m = 0; m < RL; ++m) {
-        const int row = lane + 64 * m;
-#pragma unroll
-        for (int q = 0; q < CW / 4; ++q) {
-          const float4 v = *reinterpret_cast<const float4*>(&chunk[row * CS + 4 * q]);
-          x[m][4 * q] = v.x;
-          x[m][4 * q + 1] = v.y;
-          x[m][4 * q + 2] = v.z;
-          x[m][4 * q + 3] = v.w;
-        }
-        rd[m] = rstep[row] >= 0;
-      }
-#pragma unroll
-      for (int kq = 0; kq < CW; ++kq) {
-        const int k = k0 + kq;
-        // rank: the bits of |a| (ordered as |a|), then -1 for NaN (below
-        // every number), -2 for a row already chosen
-        int f[RL], fl = -2;
+#pragma unroll 1
+    for (int ch = 0; ch < NC; ++ch) {
+      const int k0 = CW * ch;
+      float* const cc = chunk[ch & 1];
+      if (wv == 0) {
+        __builtin_amdgcn_s_setprio(3);
+        // ---- the chunk's pivot steps
+        float x[RL][CW];
+        int on[RL], mine = 0;   // on: all bits while the row has not been chosen, else 0
+        bool fine = true;
 #pragma unroll
         for (int m = 0; m < RL; ++m) {
-          const int vb = __float_as_int(x[m][kq]) & 0x7fffffff;
-          f[m] = rd[m] ? -2 : (vb > 0x7f800000 ? -1 : vb);
-          fl = f[m] > fl ? f[m] : fl;
-        }
-        const int fm = wave64_max(fl);
-        // the lowest row of rank fm: the first m with a hit, its lowest lane
-        // (some row is always left, so fm >= -1 and a hit exists)
-        int pm = 0;
-        uint64_t hit = 0;
+          const int row = lane + 64 * m;
 #pragma unroll
-        for (int m = RL - 1; m >= 0; --m) {
-          const uint64_t bm = __ballot(f[m] == fm);
-          if (bm) {
-            hit = bm;
-            pm = m;
+          for (int q = 0; q < CW / 4; ++q) {
+            const float4 v = *reinterpret_cast<const float4*>(&cc[row * CS + 4 * q]);
+            x[m][4 * q] = v.x;
+            x[m][4 * q + 1] = v.y;
+            x[m][4 * q + 2] = v.z;
+            x[m][4 * q + 3] = v.w;
           }
+          on[m] = rstep[row] < 0 ? -1 : 0;
         }
-        const int pl = hit ? (int)__builtin_ctzll(hit) : 0, p = pl + 64 * pm;
-        // the pivot row from column kq on: lane pl puts its rows out, the wave
-        // reads row pm back (the buffer is rewritten only after these reads)
-        if (lane == pl) {
 #pragma unroll
-          for (int m = 0; m < RL; ++m)
+        for (int kq = 0; kq < CW; ++kq) {
+          // rank: the bits of |a| (ordered as |a|), then those of -2.0 for NaN
+          // (below every number), the lowest for a row already chosen
+          int f[RL], fl = INT32_MIN;
 #pragma unroll
-            for (int q = 0; q < CW / 4; ++q)
-              if (q >= kq / 4)
-                *reinterpret_cast<float4*>(&prbuf[m * CW + 4 * q]) =
-                    make_float4(x[m][4 * q], x[m][4 * q + 1], x[m][4 * q + 2], x[m][4 * q + 3]);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        float pr[CW];
-#pragma unroll
-        for (int q = 0; q < CW / 4; ++q) {
-          if (q >= kq / 4) {
-            const float4 v = *reinterpret_cast<const float4*>(&prbuf[pm * CW + 4 * q]);
-            pr[4 * q] = v.x;
-            pr[4 * q + 1] = v.y;
-            pr[4 * q + 2] = v.z;
-            pr[4 * q + 3] = v.w;
+          for (int m = 0; m < RL; ++m) {
+            f[m] = min(__float_as_int(fmaxf(fabsf(x[m][kq]), -2.0f)), on[m] ^ INT32_MIN);
+            fl = max(fl, f[m]);
           }
-        }
-        const float pv = pr[kq];
-        const bool ok = pv != 0.0f && pv == pv;
+          const int fm = wave64_max(fl);
+          // the lowest row of rank fm: the first m with a hit, its lowest lane (some
+          // row is always left, so a hit exists); its values from column kq on go to
+          // scalar registers
+          float pr[CW];
+          int p = 0;
+          auto take = [&](auto place, uint64_t hit) __attribute__((always_inline)) {
+            constexpr int m = decltype(place)::value;
+            const int pl = hit ? (int)__builtin_ctzll(hit) : 0;
+            p = pl + 64 * m;
 #pragma unroll
-        for (int m = 0; m < RL; ++m) rd[m] = rd[m] || (m == pm && lane == pl);
-        if (lane == 0) {
-          prow[k] = p;
-          rstep[p] = k;
-          if (!ok) bad = 1;
-        }
-        // (recip is the same in every lane: the division runs only for a subnormal pivot)
-        const bool recip = fabsf(pv) >= 0x1p-126f;
-        const float rp = 1.0f / pv;
+            for (int c = 0; c < CW; ++c)
+              if (c >= kq) pr[c] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x[m][c]), pl));
+            on[m] = lane == pl ? 0 : on[m];
+          };
+          uint64_t hit[RL];
 #pragma unroll
-        for (int m = 0; m < RL; ++m) {
-          float li;
-          if (recip)
-            li = (!rd[m] && ok) ? x[m][kq] * rp : 0.0f;
-          else
-            li = (!rd[m] && ok) ? x[m][kq] / pv : 0.0f;
-          lz[(lane + 64 * m) * CS + kq] = li;
-          if (!rd[m] && ok) x[m][kq] = li;
+          for (int m = 0; m < RL; ++m) hit[m] = __ballot(f[m] == fm);
+          if (hit[0] | hit[1]) {
+            if (hit[0]) take(std::integral_constant<int, 0>{}, hit[0]);
+            else take(std::integral_constant<int, 1>{}, hit[1]);
+          } else {
+            if (hit[2]) take(std::integral_constant<int, 2>{}, hit[2]);
+            else take(std::integral_constant<int, 3>{}, hit[3]);
+          }
+          const float pv = pr[kq];
+          mine = lane == kq ? p : mine;   // lane q keeps step q's row
+          // a zero or NaN pivot spoils the block, which the caller then restores
+          fine = fine && pv != 0.0f && pv == pv;
+          float l[RL];
+          // (the same in every lane: the divisions run only for a subnormal pivot)
+          if (__builtin_expect(fabsf(pv) >= 0x1p-126f, 1)) {
+            const float rp = 1.0f / pv;
+#pragma unroll
+            for (int m = 0; m < RL; ++m) l[m] = x[m][kq] * rp;
+          } else {
+#pragma unroll
+            for (int m = 0; m < RL; ++m) l[m] = x[m][kq] / pv;
+          }
+#pragma unroll
+          for (int m = 0; m < RL; ++m) {   // rows already chosen keep their values
+            const int lb = __float_as_int(l[m]) & on[m];
+            x[m][kq] = __int_as_float(lb | (__float_as_int(x[m][kq]) & ~on[m]));
+            l[m] = __int_as_float(lb);
+          }
 #pragma unroll
           for (int c = 0; c < CW; ++c)
-            if (c > kq) x[m][c] -= li * pr[c];
+            if (c > kq) {
+#pragma unroll
+              for (int m = 0; m < RL; ++m) x[m][c] -= l[m] * pr[c];
+            }
         }
-      }
-#pragma unroll
-      for (int m = 0; m < RL; ++m)
-#pragma unroll
-        for (int q = 0; q < CW / 4; ++q)
-          *reinterpret_cast<float4*>(&chunk[(lane + 64 * m) * CS + 4 * q]) =
-              make_float4(x[m][4 * q], x[m][4 * q + 1], x[m][4 * q + 2], x[m][4 * q + 3]);
-#pragma unroll
-      for (int i = 0; i < RI; ++i)
-#pragma unroll
-        for (int j = 0; j < RJ; ++j) a[i][j] = park[(i * RJ + j) * 64 + lane];
-    }
-    __syncthreads();
-    // ---- the chunk applied to the later columns: the rest of group jg when
-    // the chunk is its first half (tx >= CW), and the groups after jg
-    if (mine) {
-#pragma unroll
-      for (int j = 0; j < RJ; ++j)
-        if (j == jg) {
-#pragma unroll
-          for (int i = 0; i < RI; ++i) a[i][j] = chunk[(ty + TY * i) * CS + cx];
+        if (lane < CW) {
+          prow[k0 + lane] = mine;
+          rstep[mine] = k0 + lane;
         }
-    }
-    const bool later_half = h == 0 && tx >= CW;
+        if (lane == 0 && !fine) bad = 1;
 #pragma unroll
-    for (int i = 0; i < RI; ++i) {
-      const int s = rstep[ty + TY * i] - k0;
-      if (s >= 0 && s < CW) {
+        for (int m = 0; m < RL; ++m)
 #pragma unroll
-        for (int j = 0; j < RJ; ++j)
-          if (j > jg || (j == jg && later_half)) ubuf[s * DB + tx + TX * j] = a[i][j];
+          for (int q = 0; q < CW / 4; ++q)
+            *reinterpret_cast<float4*>(&cc[(lane + 64 * m) * CS + 4 * q]) =
+                make_float4(x[m][4 * q], x[m][4 * q + 1], x[m][4 * q + 2], x[m][4 * q + 3]);
+        __builtin_amdgcn_s_setprio(0);
       }
-    }
-    __syncthreads();
-    if (t < DB - k0 - CW) {
-      // U12 column c: pivot row s minus the earlier pivots' multiples, in step order
-      const int c = k0 + CW + t;
-      float u[CW];
+      __syncthreads();
+      // U12 column c: pivot row s minus the earlier pivots' multiples, in step
+      // order (the multipliers are here before the rows are)
+      float lt[CW][CW];
 #pragma unroll
-      for (int s = 0; s < CW; ++s) {
-        const float* ls = &chunk[prow[k0 + s] * CS];
-        float v = ubuf[s * DB + c];
+      for (int s = 1; s < CW; ++s) {
+        const float* ls = &cc[prow[k0 + s] * CS];
 #pragma unroll
         for (int q = 0; 4 * q < s; ++q) {
-          const float4 l4 = *reinterpret_cast<const float4*>(ls + 4 * q);
-          const float lv[4] = {l4.x, l4.y, l4.z, l4.w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (4 * q + e < s) v -= lv[e] * u[4 * q + e];
+          const float4 v = *reinterpret_cast<const float4*>(ls + 4 * q);
+          lt[s][4 * q] = v.x;
+          lt[s][4 * q + 1] = v.y;
+          lt[s][4 * q + 2] = v.z;
+          lt[s][4 * q + 3] = v.w;
         }
-        u[s] = v;
-        ubuf[s * DB + c] = v;
+      }
+      __syncthreads();
+      if (u < DB - k0 - CW) {
+        const int c = k0 + CW + u;
+        float y[CW];
+#pragma unroll
+        for (int s = 0; s < CW; ++s) y[s] = ubuf[s * DB + c];
+#pragma unroll
+        for (int s = 0; s < CW; ++s) {
+          ubuf[s * DB + c] = y[s];
+#pragma unroll
+          for (int r = s + 1; r < CW; ++r) y[r] -= lt[r][s] * y[s];
+        }
+        // (every entry of P was read before the first chunk)
+        float* pu = P + (int64_t)k0 * ld + c;
+#pragma unroll
+        for (int s = 0; s < CW; ++s) pu[s * ld] = y[s];
+      }
+      __syncthreads();
+      __syncthreads();
+    }
+    // row r of the block goes to position invp[r]; position k moves in from
+    // block row prow[k] when they differ (moves numbered in position order)
+    const int src = prow[u];
+    const bool moved = src != u;
+    const uint64_t mb = __ballot(moved);
+    invp[src] = u;
+    ipiv[u] = src;
+    if (lane == 0) nmove[wv] = (int)__popcll(mb);
+    if (u == 0) {
+      bfirst = bpairs && bappend ? bpairs[0] : 0;
+      // the block column's first block starts the outcome word afresh
+      if (bappend) {
+        if (bad) atomicOr(fail, 1);
+      } else {
+        *fail = bad ? 1 : 0;
       }
     }
     __syncthreads();
+    {
+      int idx = (int)__popcll(mb & ((1ull << lane) - 1)), total = 0;
+#pragma unroll
+      for (int v = 0; v < DB / 64; ++v) {
+        idx += v < wv ? nmove[v] : 0;
+        total += nmove[v];
+      }
+      if (moved) {
+        pairs[1 + 2 * idx] = base + u;
+        pairs[2 + 2 * idx] = base + src;
+        if (bpairs) {
+          bpairs[1 + 2 * (bfirst + idx)] = base + u;
+          bpairs[2 + 2 * (bfirst + idx)] = base + src;
+        }
+      }
+      if (u == 0) {
+        pairs[0] = total;
+        if (bpairs) bpairs[0] = bfirst + total;
+      }
+    }
+    return;
+  }
+  f32x16 a[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a[j][r] = P[(int64_t)(row0 + 8 * (r >> 2) + (r & 3)) * ld + 32 * j + li];
+  if (li < CW) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) chunk[0][(row0 + 8 * (r >> 2) + (r & 3)) * CS + li] = a[0][r];
+  }
+  __syncthreads();   // (every entry of P has been read: rows of U are written below)
 #pragma unroll 1
-    for (int q = 0; q < CW / 4; ++q) {
-      float l4[RI][4];
+  for (int ch = 0;; ++ch) {
+    const int k0 = CW * ch, jg = ch >> 1, h = ch & 1;
+    const float* const cc = chunk[ch & 1];
+    if (ch > 0) {
+      // ---- the last chunk's own columns back into their tile, and its L21 U12
+      // off the tiles after this chunk's
+      const float* const cp = chunk[(ch & 1) ^ 1];
 #pragma unroll
-      for (int i = 0; i < RI; ++i) {
-        const float4 v = *reinterpret_cast<const float4*>(&lz[(ty + TY * i) * CS + 4 * q]);
-        l4[i][0] = v.x;
-        l4[i][1] = v.y;
-        l4[i][2] = v.z;
-        l4[i][3] = v.w;
+      for (int j = 0; j < NJ; ++j)
+        if (j == (ch - 1) >> 1 && (li / CW) != h) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) a[j][r] = cp[(row0 + 8 * (r >> 2) + (r & 3)) * CS + li % CW];
+        }
+      if (ch == NC) break;
+      float l[CW / 2];
+#pragma unroll
+      for (int s = 0; s < CW / 2; ++s) l[s] = -cp[(32 * wv + li) * CS + 2 * s + hk];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (j > jg) {
+#pragma unroll
+          for (int s = 0; s < CW / 2; ++s)
+            a[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(l[s], ubuf[(2 * s + hk) * DB + 32 * j + li], a[j], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    // ---- the chunk's pivot rows on the later columns, into ubuf
+    {
+      int rs[16];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int4 v = *reinterpret_cast<const int4*>(&rstep[row0 + 8 * q]);
+        rs[4 * q] = v.x;
+        rs[4 * q + 1] = v.y;
+        rs[4 * q + 2] = v.z;
+        rs[4 * q + 3] = v.w;
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
+      for (int r = 0; r < 16; ++r) {
+        const int s = rs[r] - k0;
+        if (s >= 0) {
 #pragma unroll
-        for (int j = 0; j < RJ; ++j)
-          if (j > jg || (j == jg && later_half)) {
-            const float u = ubuf[(4 * q + e) * DB + tx + TX * j];
-#pragma unroll
-            for (int i = 0; i < RI; ++i) a[i][j] -= l4[i][e] * u;
-          }
+          for (int j = 0; j < NJ; ++j) ubuf[s * DB + 32 * j + li] = a[j][r];   // (columns before the chunk are not used)
+        }
       }
     }
-    __syncthreads();   // chunk, lz and ubuf are rewritten by the next chunk
-  }
-  // row r of the block goes to position invp[r]; position k moves in from
-  // block row prow[k] when they differ (moves numbered in position order)
-  const bool moved = t < DB && prow[t] != t;
-  const uint64_t mb = __ballot(moved);
-  if (t < DB) {
-    invp[prow[t]] = t;
-    ipiv[t] = prow[t];
-    if (lane == 0) nmove[wv] = (int)__popcll(mb);
-  }
-  if (t == 0) {
-    bfirst = bpairs && bappend ? bpairs[0] : 0;
-    // the block column's first block starts the outcome word afresh
-    if (bappend) {
-      if (bad) atomicOr(fail, 1);
-    } else {
-      *fail = bad ? 1 : 0;
+    __syncthreads();
+    __syncthreads();
+    // ---- the tile with the next chunk: L21 U12 off it, the chunk out to LDS
+    {
+      const int jn = (ch + 1) >> 1;
+      float l[CW / 2];
+#pragma unroll
+      for (int s = 0; s < CW / 2; ++s) l[s] = -cc[(32 * wv + li) * CS + 2 * s + hk];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (j == jn) {
+#pragma unroll
+          for (int s = 0; s < CW / 2; ++s)
+            a[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(l[s], ubuf[(2 * s + hk) * DB + 32 * j + li], a[j], 0, 0, 0);
+        }
+      float* const cn = chunk[(ch & 1) ^ 1];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (j == jn && (li / CW) != h) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) cn[(row0 + 8 * (r >> 2) + (r & 3)) * CS + li % CW] = a[j][r];
+        }
     }
+    __syncthreads();
   }
   __syncthreads();
-  if (t < DB) {
-    int idx = (int)__popcll(mb & ((1ull << lane) - 1)), total = 0;
+  // each row up to the end of the chunk that chose it (the rest is U12)
 #pragma unroll
-    for (int v = 0; v < DB / 64; ++v) {
-      idx += v < wv ? nmove[v] : 0;
-      total += nmove[v];
-    }
-    if (moved) {
-      pairs[1 + 2 * idx] = base + t;
-      pairs[2 + 2 * idx] = base + prow[t];
-      if (bpairs) {
-        bpairs[1 + 2 * (bfirst + idx)] = base + t;
-        bpairs[2 + 2 * (bfirst + idx)] = base + prow[t];
-      }
-    }
-    if (t == 0) {
-      pairs[0] = total;
-      if (bpairs) bpairs[0] = bfirst + total;
-    }
-  }
+  for (int r = 0; r < 16; ++r) {
+    const int row = invp[row0 + 8 * (r >> 2) + (r & 3)];
 #pragma unroll
-  for (int i = 0; i < RI; ++i) {
-    const int64_t row = invp[ty + TY * i];
-#pragma unroll
-    for (int j = 0; j < RJ; ++j) P[row * ld + tx + TX * j] = a[i][j];
+    for (int j = 0; j < NJ; ++j)
+      if (32 * j + li < (row / CW + 1) * CW) P[(int64_t)row * ld + 32 * j + li] = a[j][r];
   }
 }
 
@@ -1171,7 +1212,7 @@ void optimistic_block(float* P, int64_t lda, int64_t rows, const float* src21, i
                       float* linv = nullptr, int64_t linv_ld = 0, int32_t* bpairs = nullptr, int bappend = 0,
                       float* linv_init = nullptr) {
   MixedCtx& mx = tl_mix;
-  hipLaunchKernelGGL(diag_getf2_kernel<DIAG_TY>, dim3(1), dim3(DIAG_TY * 32), 0, s, P, lda, ipiv, base, mx.pfail,
+  hipLaunchKernelGGL(diag_getf2_kernel, dim3(1), dim3(DIAG_NT), 0, s, P, lda, ipiv, base, mx.pfail,
                      pairs, bpairs, bappend);
   ZH_LAUNCH_CHECK();
   if (linv_init) {   // the block column's whole L11^-1 buffer starts as the identity
