@@ -71,3 +71,37 @@ def test_many_workgroup_rounds_match_between_tiles(zh, torch_cuda):
             out.append(c)
         torch.cuda.synchronize()
         assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("transa,transb", [(111, 111), (112, 111), (111, 112), (112, 112)])
+@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (-1.0, 1.0), (0.5, 2.0)])
+def test_fp32_load_unit_kernel(zh, torch_cuda, transa, transb, alpha, beta):
+    """FP32 products on the load unit: ragged tiles in both directions (the last
+    four rows or columns alone in theirs), one slab and several. The same bits as
+    with the load-unit kernel off, and within k u of the sum of the products'
+    magnitudes (u = 2^-24, gamma_k) of the FP64 product."""
+    torch = torch_cuda
+    import ctypes
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for m, n, k in ((2048, 2048, 32), (2436, 2564, 96), (4100, 2052, 160)):
+        g = torch.Generator(device="cuda")
+        g.manual_seed(m + k)
+        sa = (k, m) if transa == 111 else (m, k)     # column-major storage seen as rows
+        sb = (n, k) if transb == 111 else (k, n)
+        a, b, c0 = (torch.rand(x, dtype=torch.float32, device="cuda", generator=g) - 0.5 for x in (sa, sb, (n, m)))
+        out = []
+        for on in (0, 1):
+            c = c0.clone()
+            was = zh.zmlhip_set_gemm_lds_dma(on)
+            try:
+                assert zh.zmlhip_sgemm(COL, transa, transb, m, n, k, alpha, P(a), sa[1], P(b), sb[1], beta, P(c), m, s) == 0
+            finally:
+                zh.zmlhip_set_gemm_lds_dma(was)
+            out.append(c)
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], out[1])
+        A = (a.t() if transa == 111 else a).double()     # m x k
+        Bm = (b.t() if transb == 111 else b).double()    # k x n
+        ref = alpha * (A @ Bm) + beta * c0.t().double()
+        mag = abs(alpha) * (A.abs() @ Bm.abs()) + abs(beta) * c0.t().double().abs()
+        assert bool(((out[1].t().double() - ref).abs() <= (k + 3) * 2.0 ** -24 * mag).all())

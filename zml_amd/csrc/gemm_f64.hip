@@ -11,9 +11,9 @@
 //
 // Two kernels, with the same order of operations for every element of C (the same
 // bits), chosen in gemm_cm:
-//  - gemm_dma_f64_kernel (FP64, whole k-slabs, 16-byte aligned operand columns):
-//    128 x 128 tiles whose operand slabs go from global memory to LDS by the load
-//    unit; 71 TF/s at 4096^3 and above on MI355X;
+//  - gemm_dma_kernel (whole k-slabs, 16-byte aligned operand columns): 128 x 128
+//    tiles whose operand slabs go from global memory to LDS by the load unit; 71
+//    TF/s FP64, 122 TF/s FP32 at 4096^3 on MI355X;
 //  - gemm_small_kernel (every shape, FP64 and FP32): 64 x 64 tiles staged through
 //    registers, four workgroups per CU, with k split over workgroups where even
 //    these are few.
@@ -59,7 +59,7 @@ template <> struct Mfma<float> {
 };
 
 constexpr int BM = 128, BN = 128, BK = 16, PAD = 2;
-constexpr int LDA_S = BM + PAD, LDB_S = BN + PAD;
+constexpr int LDA_S = BM + PAD;
 constexpr int NT = 256;
 
 // Maps the linear workgroup id to a (tile_m, tile_n) pair: consecutive ids
@@ -247,89 +247,110 @@ splitk_sum_kernel(int64_t m, int64_t n, int nz, const T* __restrict__ part, T al
   *c = beta == T(0) ? v : (beta == T(1) ? *c + v : beta * *c + v);
 }
 
-// ---- FP64 with the operand slabs moved global -> LDS by the load unit
+// ---- 128 x 128 tiles with the operand slabs moved global -> LDS by the load unit
 //
 // MFMA order and epilogue as gemm_small_kernel (the results are identical bit for
 // bit) on 128 x 128 tiles (four waves of 64 x 64); every thread issues 8 global_load_lds_dwordx4
-// per 16-wide k-slab: each lane's 16 bytes land in LDS at 16 x its lane id
+// per slab of 128 bytes along k (16 doubles, 32 floats): each lane's 16 bytes land in LDS at 16 x its lane id
 // after the instruction's (wave-uniform) base, without passing through VGPRs
 // and without ds_write instructions. Two LDS buffers: slab kt + 1 is in flight
 // while slab kt is multiplied; one barrier per slab, after each thread's own
 // loads have landed (vmcnt 0).
-// Slab layouts in LDS (doubles):
-//  - operand contiguous along m (A) or n (op(B) = B^T): 16 k-rows of 128
+// Slab layouts in LDS:
+//  - operand contiguous along m (A) or n (op(B) = B^T), FP64: 16 k-rows of 128
 //    elements, k-row l at l * LDA_S; a wave instruction moves one k-row (lane:
 //    elements 2 lane, 2 lane + 1, so the m / n extent must be even);
-//  - operand contiguous along k: 128 columns of 16, column c at 16 c, k pairs
-//    stored at slot pair ^ sw(c), sw(c) = (c ^ c >> 3) & 7, so that the 16
+//  - the same, FP32: 32 k-rows of 128 floats, an instruction moves two (32 lanes
+//    of 4 floats each, so the extent must be a multiple of 4); an odd row has its
+//    16-float groups exchanged in pairs, so that the four rows a fragment reads
+//    lie in both halves of the LDS banks;
+//  - operand contiguous along k: 128 columns of 128 bytes, its eight 16-byte chunks
+//    stored at slot chunk ^ sw(c), sw(c) = (c ^ c >> 3) & 7, so that the 16
 //    lanes reading one k of 16 consecutive columns hit distinct LDS banks; a
-//    wave instruction moves 8 columns (lane 8 jj + s: column 8 q + jj, the pair
+//    wave instruction moves 8 columns (lane 8 jj + s: column 8 q + jj, the chunk
 //    s ^ sw).
 // For the update form with alpha = -1 the A fragments are negated after their
 // LDS reads (gemm_small_kernel negates B before storing it): either
 // way every product enters the accumulator as fl(c - a b).
-constexpr int DBK = 16;
-constexpr int DSLAB = DBK * LDA_S;   // doubles per operand buffer (>= 128 x 16)
+// FP32 reaches 122 TF/s at 4096^3 (1127 us against 1362 us on 64 x 64 tiles; a large
+// library product reaches 148 on this card): bound by the matrix cores and, with two
+// workgroups a CU, the wait at each slab's barrier.
+template <typename T> constexpr int kDmaK = 128 / (int)sizeof(T);                   // k of a slab
+template <typename T> constexpr int kDmaSlab = sizeof(T) == 8 ? 16 * LDA_S : 4096;   // elements per operand buffer
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
 
-__device__ __forceinline__ void lds_dma16(const double* g, double* l) {
-  __builtin_amdgcn_global_load_lds((const void*)g, (lds_void_ptr)l, 16, 0, 0);
+__device__ __forceinline__ void lds_dma16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds(g, (lds_void_ptr)l, 16, 0, 0);
+}
+__device__ __forceinline__ double flip(double v, bool neg) {
+  return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, v) ^ (neg ? 0x8000000000000000ull : 0ull));
+}
+__device__ __forceinline__ float flip(float v, bool neg) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) ^ (neg ? 0x80000000u : 0u));
 }
 
 // One operand's slab mover and fragment reader. MNC: contiguous along m / n.
-template <bool MNC>
+template <typename T, bool MNC>
 struct DmaOperand {
-  const double* p[4];   // per-thread source of each of the thread's 4 instructions (k0 = 0)
+  static constexpr bool kF32 = sizeof(T) == 4;
+  static constexpr int CE = 16 / (int)sizeof(T);   // elements of a 16-byte chunk
+  const T* p[4];        // per-thread source of each of the thread's 4 instructions (k0 = 0)
   int64_t ld;
-  int o[4];             // K-contiguous: LDS offset of fragment x at ks = 0
-  int base;             // MN-contiguous: LDS offset of fragment 0 at ks = 0
+  int o[4];             // LDS offset of fragment x at ks = 0
 
-  __device__ __forceinline__ void init(const double* X, int64_t ldx, int64_t mn0, int64_t mn, int wave, int lane,
+  __device__ __forceinline__ void init(const T* X, int64_t ldx, int64_t mn0, int64_t mn, int wave, int lane,
                                        int w, int lr, int lk) {
     ld = ldx;
     if (MNC) {
-      const int64_t e = mn0 + 2 * lane < mn ? mn0 + 2 * lane : mn - 2;
+      const int rr = kF32 ? lane >> 5 : 0;   // row of the instruction's two
+      const int64_t e0 = mn0 + CE * (kF32 ? (lane & 31) ^ (4 * rr) : lane), e = e0 < mn ? e0 : mn - CE;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) p[c] = X + e + (int64_t)(wave + 4 * c) * ldx;
-      base = w * 64 + lr + lk * LDA_S;
+      for (int c = 0; c < 4; ++c) p[c] = X + e + (int64_t)((kF32 ? 2 : 1) * (wave + 4 * c) + rr) * ldx;
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        o[x] = w * 64 + lr + (kF32 ? lk * 128 + 16 * (x ^ (lk & 1)) : lk * LDA_S + 16 * x);
     } else {
       const int jj = lane >> 3, s = lane & 7;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const int q = wave + 4 * c;
         const int64_t col = mn0 + 8 * q + jj < mn ? mn0 + 8 * q + jj : mn - 1;
-        p[c] = X + 2 * (s ^ ((jj ^ q) & 7)) + col * ldx;
+        p[c] = X + CE * (s ^ ((jj ^ q) & 7)) + col * ldx;
       }
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const int c = w * 64 + 16 * x + lr;
-        o[x] = c * DBK + 2 * ((lk >> 1) ^ ((c ^ (c >> 3)) & 7)) + (lk & 1);
+        o[x] = c * kDmaK<T> + CE * ((lk / CE) ^ ((c ^ (c >> 3)) & 7)) + lk % CE;
       }
     }
   }
-  __device__ __forceinline__ void issue(int64_t k0, double* buf, int wave) const {
+  __device__ __forceinline__ void issue(int64_t k0, T* buf, int wave) const {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      if (MNC) lds_dma16(p[c] + k0 * ld, buf + (wave + 4 * c) * LDA_S);
-      else lds_dma16(p[c] + k0, buf + (wave + 4 * c) * 128);
+      if (MNC) lds_dma16(p[c] + k0 * ld, buf + (wave + 4 * c) * (kF32 ? 256 : LDA_S));
+      else lds_dma16(p[c] + k0, buf + (wave + 4 * c) * 8 * kDmaK<T>);
     }
   }
   // fragment x (16 elements along m / n) at k = 4 ks + lk
-  __device__ __forceinline__ double frag(const double* buf, int ks, int x) const {
-    return MNC ? buf[base + 4 * ks * LDA_S + 16 * x] : buf[o[x] ^ (4 * ks)];
+  __device__ __forceinline__ T frag(const T* buf, int ks, int x) const {
+    return MNC ? buf[o[x] + 4 * ks * (kF32 ? 128 : LDA_S)] : buf[o[x] ^ (4 * ks)];
   }
 };
 
-template <bool TA, bool TB>
+// init: the update form accumulates onto C itself (as the other kernel does);
+// otherwise the products are summed first and C added once.
+template <typename T, bool TA, bool TB>
 __global__ void __launch_bounds__(NT, 2)
-gemm_dma_f64_kernel(int64_t m, int64_t n, int64_t k, double alpha, const double* __restrict__ A, int64_t lda,
-                    const double* __restrict__ B, int64_t ldb, double beta, double* __restrict__ C, int64_t ldc,
-                    int tri, int64_t tri_tiles) {
-  __shared__ __attribute__((aligned(16))) double As0[DSLAB];
-  __shared__ __attribute__((aligned(16))) double As1[DSLAB];
-  __shared__ __attribute__((aligned(16))) double Bs0[DSLAB];
-  __shared__ __attribute__((aligned(16))) double Bs1[DSLAB];
+gemm_dma_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict__ A, int64_t lda,
+                const T* __restrict__ B, int64_t ldb, T beta, T* __restrict__ C, int64_t ldc,
+                int tri, int64_t tri_tiles, int init) {
+  typedef typename Mfma<T>::acc acc_t;
+  constexpr int DBK = kDmaK<T>;
+  __shared__ __attribute__((aligned(16))) T As0[kDmaSlab<T>];
+  __shared__ __attribute__((aligned(16))) T As1[kDmaSlab<T>];
+  __shared__ __attribute__((aligned(16))) T Bs0[kDmaSlab<T>];
+  __shared__ __attribute__((aligned(16))) T Bs1[kDmaSlab<T>];
 
   const int64_t ntm = (m + BM - 1) / BM, ntn = (n + BN - 1) / BN;
   int64_t tm, tn;
@@ -344,21 +365,21 @@ gemm_dma_f64_kernel(int64_t m, int64_t n, int64_t k, double alpha, const double*
   const int wm = wave & 1, wn = wave >> 1;
   const int lr = lane & 15, lk = lane >> 4;
 
-  DmaOperand<!TA> opa;
-  DmaOperand<TB> opb;
+  DmaOperand<T, !TA> opa;
+  DmaOperand<T, TB> opb;
   opa.init(A, lda, row0, m, wave, lane, wm, lr, lk);
   opb.init(B, ldb, col0, n, wave, lane, wn, lr, lk);
 
-  const bool cinit = beta == 1.0 && (alpha == 1.0 || alpha == -1.0);
-  const unsigned long long sgn = (cinit && alpha == -1.0) ? 0x8000000000000000ull : 0ull;
+  const bool cinit = init && beta == T(1) && (alpha == T(1) || alpha == T(-1));
+  const bool neg = cinit && alpha == T(-1);
   auto c_ok = [&](int64_t i, int64_t j) {
     return i < m && j < n && !(tri == kLower && i < j) && !(tri == kUpper && i > j);
   };
-  d4 acc[4][4];
+  acc_t acc[4][4];
 #pragma unroll
   for (int x = 0; x < 4; ++x)
 #pragma unroll
-    for (int y = 0; y < 4; ++y) acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int y = 0; y < 4; ++y) acc[x][y] = acc_t{T(0), T(0), T(0), T(0)};
   if (cinit) {
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
@@ -367,25 +388,24 @@ gemm_dma_f64_kernel(int64_t m, int64_t n, int64_t k, double alpha, const double*
       for (int y = 0; y < 4; ++y)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int64_t j = col0 + wn * 64 + 16 * y + Mfma<double>::col(lk, r);
+          const int64_t j = col0 + wn * 64 + 16 * y + Mfma<T>::col(lk, r);
           if (c_ok(i, j)) acc[x][y][r] = C[i + j * ldc];
         }
     }
   }
 
-  auto compute = [&](const double* as, const double* bs) {
+  auto compute = [&](const T* as, const T* bs) {
 #pragma unroll
     for (int ks = 0; ks < DBK / 4; ++ks) {
-      double av[4], bv[4];
+      T av[4], bv[4];
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
-        av[x] = __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, opa.frag(as, ks, x)) ^ sgn);
+      for (int x = 0; x < 4; ++x) av[x] = flip(opa.frag(as, ks, x), neg);
 #pragma unroll
       for (int y = 0; y < 4; ++y) bv[y] = opb.frag(bs, ks, y);
 #pragma unroll
       for (int x = 0; x < 4; ++x)
 #pragma unroll
-        for (int y = 0; y < 4; ++y) acc[x][y] = Mfma<double>::step(bv[y], av[x], acc[x][y]);
+        for (int y = 0; y < 4; ++y) acc[x][y] = Mfma<T>::step(bv[y], av[x], acc[x][y]);
     }
   };
   // vmcnt(0), expcnt and lgkmcnt left at their maxima
@@ -419,25 +439,25 @@ gemm_dma_f64_kernel(int64_t m, int64_t n, int64_t k, double alpha, const double*
       for (int y = 0; y < 4; ++y)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int64_t j = col0 + wn * 64 + 16 * y + Mfma<double>::col(lk, r);
+          const int64_t j = col0 + wn * 64 + 16 * y + Mfma<T>::col(lk, r);
           if (c_ok(i, j)) C[i + j * ldc] = acc[x][y][r];
         }
     }
     return;
   }
-  const bool need_c = beta != 0.0;
+  const bool need_c = beta != T(0);
 #pragma unroll
   for (int x = 0; x < 4; ++x) {
     const int64_t i = row0 + wm * 64 + 16 * x + lr;
     bool ok[4][4];
-    double cv[4][4];
+    T cv[4][4];
 #pragma unroll
     for (int y = 0; y < 4; ++y) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t j = col0 + wn * 64 + 16 * y + Mfma<double>::col(lk, r);
+        const int64_t j = col0 + wn * 64 + 16 * y + Mfma<T>::col(lk, r);
         ok[y][r] = c_ok(i, j);
-        cv[y][r] = (need_c && ok[y][r]) ? C[i + j * ldc] : 0.0;
+        cv[y][r] = (need_c && ok[y][r]) ? C[i + j * ldc] : T(0);
       }
     }
 #pragma unroll
@@ -445,24 +465,25 @@ gemm_dma_f64_kernel(int64_t m, int64_t n, int64_t k, double alpha, const double*
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         if (!ok[y][r]) continue;
-        const int64_t j = col0 + wn * 64 + 16 * y + Mfma<double>::col(lk, r);
-        const double v = alpha * acc[x][y][r];
-        C[i + j * ldc] = beta == 0.0 ? v : (beta == 1.0 ? cv[y][r] + v : beta * cv[y][r] + v);
+        const int64_t j = col0 + wn * 64 + 16 * y + Mfma<T>::col(lk, r);
+        const T v = alpha * acc[x][y][r];
+        C[i + j * ldc] = beta == T(0) ? v : (beta == T(1) ? cv[y][r] + v : beta * cv[y][r] + v);
       }
     }
   }
 }
 
-// Whether gemm_dma_f64_kernel takes the product: whole 16-wide k-slabs, 16-byte
-// aligned operand columns, and an even extent along each operand's contiguous
-// m / n direction.
-inline bool dma_f64_ok(bool ta, bool tb, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda,
-                       const void* b, int64_t ldb) {
-  if (k < DBK || k % DBK != 0) return false;
+// Whether gemm_dma_kernel takes the product: whole k-slabs, 16-byte aligned operand
+// columns, and whole 16-byte chunks along each operand's contiguous m / n direction.
+template <typename T>
+inline bool dma_ok(bool ta, bool tb, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda,
+                   const void* b, int64_t ldb) {
+  constexpr int CE = 16 / (int)sizeof(T);
+  if (k < kDmaK<T> || k % kDmaK<T> != 0) return false;
   if ((((uintptr_t)a) | ((uintptr_t)b)) & 15) return false;
-  if ((lda | ldb) & 1) return false;
-  if (!ta && (m & 1)) return false;
-  if (tb && (n & 1)) return false;
+  if (lda % CE || ldb % CE) return false;
+  if (!ta && m % CE) return false;
+  if (tb && n % CE) return false;
   return true;
 }
 
@@ -493,15 +514,20 @@ template void scale_cm<double>(int64_t, int64_t, double, double*, int64_t, hipSt
 template void scale_cm<float>(int64_t, int64_t, float, float*, int64_t, hipStream_t, int);
 
 // 64 x 64 tiles rather than 128 x 128 ones moved by the load unit. Both run in
-// rounds over the CUs; a CU delivers 0.27 TF/s on 128 x 128 tiles (0.24 while it has
-// only one), 0.22 on 64 x 64 ones, so a round of the first costs 3.26 (3.64) rounds
-// of the second: 2048 x 2176 x 784 (272 tiles, two rounds for one tile more than a
-// CU each) 198 against 163 us, 2048^3 (256 tiles) 277 against 322 us, 2500^2 x 2512
-// 609 against 671 us.
+// rounds over the CUs, and a round of the first costs 3.26 rounds of the second in
+// FP64 (0.27 TF/s a CU on 128 x 128 tiles, 0.22 on 64 x 64 ones), 3.45 in FP32 (0.48
+// and 0.40; 3.2 to 3.6 over k = 320 .. 4096), more while a CU has only one tile
+// (3.64 and 4.0). FP64: 2048 x 2176 x 784 (272 tiles, two rounds for one tile more
+// than a CU each) 198 against 163 us, 2048^3 (256 tiles) 277 against 322 us, 2500^2 x
+// 2512 609 against 671 us. FP32: 2048 x 2176 x 768 117 against 91 us, 2048^3 186
+// against 190 us, 2500^2 x 2496 349 against 386 us, 3100 x 2900 x 3008 (575 tiles)
+// 664 against 581 us, 4096^3 1127 against 1362 us.
+template <typename T>
 static bool small_tiles(int64_t t128, int64_t t64) {
   const int64_t cus = device_cu_count();
   const int64_t r128 = (t128 + cus - 1) / cus, r64 = (t64 + cus - 1) / cus;
-  return (r128 == 1 ? 364 : 326 * r128) > 100 * r64;
+  constexpr int one = sizeof(T) == 8 ? 364 : 400, more = sizeof(T) == 8 ? 326 : 345;
+  return (r128 == 1 ? one : more * r128) > 100 * r64;
 }
 
 template <typename T>
@@ -527,6 +553,29 @@ static void small_gemm(bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alph
 }
 
 template <typename T>
+static void dma_gemm(bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda, const T* b,
+                     int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int64_t tiles, int64_t tri_tiles,
+                     int init) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(NT), 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc,
+                       tri, tri_tiles, init);
+  };
+  if (!ta && !tb) go(gemm_dma_kernel<T, false, false>);
+  else if (ta && !tb) go(gemm_dma_kernel<T, true, false>);
+  else if (!ta && tb) go(gemm_dma_kernel<T, false, true>);
+  else go(gemm_dma_kernel<T, true, true>);
+  ZH_LAUNCH_CHECK();
+}
+
+bool gemm_f32_dma_cm(int64_t m, int64_t n, int64_t k, float alpha, const float* a, int64_t lda, const float* b,
+                     int64_t ldb, float beta, float* c, int64_t ldc, hipStream_t s) {
+  if (!gemm_dma_enabled() || !dma_ok<float>(false, false, m, n, k, a, lda, b, ldb)) return false;
+  const int64_t tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
+  dma_gemm<float>(false, false, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, 0, tiles, 0, 0);
+  return true;
+}
+
+template <typename T>
 void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda,
              const T* b, int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int split_slot) {
   if (m <= 0 || n <= 0) return;
@@ -540,16 +589,9 @@ void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, c
   const int64_t tiles = tri_tiles > 0 ? tri_tiles : ntm * ntn;
   const int64_t nsm = (m + SM - 1) / SM, nsn = (n + SM - 1) / SM;
   const int64_t stri = tri_tile_count(tri, nsm, nsn), stiles = stri > 0 ? stri : nsm * nsn;
-  if constexpr (std::is_same<T, double>::value) {
-    if (gemm_dma_enabled() && dma_f64_ok(ta, tb, m, n, k, a, lda, b, ldb) && !small_tiles(tiles, stiles)) {
-      const dim3 grid((unsigned)tiles), block(NT);
-      if (!ta && !tb) hipLaunchKernelGGL((gemm_dma_f64_kernel<false, false>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
-      else if (ta && !tb) hipLaunchKernelGGL((gemm_dma_f64_kernel<true, false>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
-      else if (!ta && tb) hipLaunchKernelGGL((gemm_dma_f64_kernel<false, true>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
-      else hipLaunchKernelGGL((gemm_dma_f64_kernel<true, true>), grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles);
-      ZH_LAUNCH_CHECK();
-      return;
-    }
+  if (gemm_dma_enabled() && dma_ok<T>(ta, tb, m, n, k, a, lda, b, ldb) && !small_tiles<T>(tiles, stiles)) {
+    dma_gemm<T>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, tiles, tri_tiles, 1);
+    return;
   }
   // k is split where the tiles leave CUs idle: about two workgroups per CU, each
   // with at least 128 of k (a split of 4 or 8 slabs no longer pays its sum)

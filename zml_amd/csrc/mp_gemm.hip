@@ -602,6 +602,8 @@ void mp_gemm_f32(int64_t m, int64_t n, int64_t K, float alpha, const float* A, i
                  const float* B, int64_t ldb, float beta, const float* rs, const float* cs, float* C,
                  int64_t ldc, hipStream_t s, int lower) {
   if (m <= 0 || n <= 0) return;
+  // row-major C = A B is column-major C^T = B^T A^T on the same memory
+  if (!rs && !cs && !lower && gemm_f32_dma_cm(n, m, K, alpha, B, ldb, A, lda, beta, C, ldc, s)) return;
   const int64_t ntm = (m + MT - 1) / MT, ntn = (n + NTL - 1) / NTL;
   const int64_t tri_tiles = lower ? tri_tile_count(kLower, ntm, ntn) : 0;
   const int64_t tiles = tri_tiles > 0 ? tri_tiles : ntm * ntn;

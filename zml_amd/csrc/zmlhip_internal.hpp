@@ -147,6 +147,10 @@ inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 template <typename T>
 void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda,
              const T* b, int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int split_slot = -1);
+// C = alpha A B + beta C (FP32, column-major, the products summed before C is added)
+// by the load-unit kernel; false, with nothing launched, for shapes it does not take.
+bool gemm_f32_dma_cm(int64_t m, int64_t n, int64_t k, float alpha, const float* a, int64_t lda, const float* b,
+                     int64_t ldb, float beta, float* c, int64_t ldc, hipStream_t s);
 template <typename T>
 void scale_cm(int64_t m, int64_t n, T beta, T* c, int64_t ldc, hipStream_t s, int tri);
 template <typename T>
