@@ -4,15 +4,16 @@
 // system the arithmetic is the one of the large mixed solves: an FP32
 // factorization and FP64 iterative refinement against the FP64 A.
 //
-// A plan sorts the systems into size buckets (n <= 32, 64, 128, 256). Every
-// bucket runs one persistent kernel whose workgroups take systems from an
-// atomic work queue; a workgroup keeps its system's FP32 factor in registers
+// A plan sorts the systems into size buckets (n <= 32, 64, 128, 256). The two
+// smaller buckets run a persistent kernel each, whose workgroups take systems from
+// an atomic work queue; a workgroup keeps its system's FP32 factor in registers
 // (a TY x TX thread grid, RI x RJ values per thread, NMAX = TY RI = TX RJ) from the
 // factorization through every refinement step, and reads the FP64 matrix
-// from HBM only for the residuals. The thread-grid shape of every bucket is
-// chosen by timing the candidate shapes on the bucket's own systems
-// (autotune), and the queue resets plus the bucket kernels are captured once
-// into a hipGraph, so that one graph launch solves the whole batch.
+// from HBM only for the residuals. The thread-grid shape is chosen by timing the
+// candidate shapes on the bucket's own systems (autotune). The two larger buckets
+// run one workgroup per system with the factor in matrix-core accumulators. The
+// queue resets plus the bucket kernels are captured once into a hipGraph, so that
+// one graph launch solves the whole batch.
 //
 // The FP32 factorization is a Gauss-Jordan inversion in place: general
 // systems pivot on the largest |a| of the column among the rows not yet
@@ -30,6 +31,7 @@
 #include <algorithm>
 #include <cmath>
 #include <memory>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/zmlhip.h"
@@ -293,27 +295,500 @@ __global__ void __launch_bounds__(TY * TX) batched_solve_kernel(BatchArgs g) {
   }
 }
 
+// ---- n <= 128 and n <= 256: the matrix in MFMA accumulators, 16 columns at a time
+//
+// ND waves hold the FP32 matrix as 32 x 32 accumulator tiles (wave w the rows
+// 32 w .. 32 w + 31 of ND tiles), and ND / 2 helper waves hold nothing. The
+// Gauss-Jordan steps go in chunks of 16 columns: helper wave 0 has the chunk in its
+// registers (rows lane + 64 m) and runs its 16 steps there, without barriers: the
+// pivot's rank through DPP, the pivot row into scalar registers, one reciprocal,
+// the other rows' update (the pivot row's own factor 1 / pivot is applied at the end
+// of the chunk). That leaves G, the chunk's columns of the result; with U the pivot
+// rows' values in the other columns before the chunk, every other column becomes
+// M + G U, pivot rows counted as zero in M: one product of inner length 16 on the
+// matrix cores. The tile with the next chunk goes first, the rest while helper wave
+// 0 runs the next steps. (A last chunk of fewer than 16 columns is filled up with
+// the identity.)
+// Refinement: the accumulator waves form inv32(A) r, the helper threads (one row
+// each) the FP64 residuals, for up to four right-hand sides in one pass over A.
+//
+// Bound by helper wave 0's chain, about 1,000 cycles a column, with one workgroup
+// on a CU at n <= 256 (its registers hold no second one): 145 of 200 us a system,
+// the rest the residuals' passes over A. 4,000 systems of order 129 .. 256: 3.16 ms,
+// 65 .. 128: 0.87 ms (one MI355X). A thread grid with 128 (64) entries a thread,
+// two barriers, a search through LDS and a rank-1 update in every column, half of
+// whose instructions moved operands between the register files, and one pass over
+// A for every right-hand side and step took 7.29 and 1.32 ms.
+constexpr int BQ = 4;   // right-hand sides refined together
+
+__device__ __forceinline__ int imax_all(int v) {   // the largest v of the wave, in every lane
+  auto step = [&](int o) { v = o > v ? o : v; };
+  step(__builtin_amdgcn_update_dpp((int)0x80000000, v, 0xb1, 0xf, 0xf, false));    // quad_perm [1,0,3,2]
+  step(__builtin_amdgcn_update_dpp((int)0x80000000, v, 0x4e, 0xf, 0xf, false));    // quad_perm [2,3,0,1]
+  step(__builtin_amdgcn_update_dpp((int)0x80000000, v, 0x124, 0xf, 0xf, false));   // row_ror:4
+  step(__builtin_amdgcn_update_dpp((int)0x80000000, v, 0x128, 0xf, 0xf, false));   // row_ror:8
+  step(__builtin_amdgcn_update_dpp((int)0x80000000, v, 0x142, 0xa, 0xf, false));   // row_bcast:15 into rows 1, 3
+  step(__builtin_amdgcn_update_dpp((int)0x80000000, v, 0x143, 0xc, 0xf, false));   // row_bcast:31 into rows 2, 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+template <int ND>
+struct TileShared {
+  static constexpr int NMAX = 32 * ND, CW = 16, CS = CW + 4, NH = ND / 2;
+  float chunk[2][NMAX * CS];   // row r of a chunk at r CS; the two together stage A at the start
+  float ubuf[CW * NMAX];       // row s: the chunk's pivot row s before the chunk
+  float cv[BQ][NMAX], yv[BQ][NMAX];
+  double xv[NMAX][BQ], rv[BQ][NMAX];
+  double red[NH][2 * BQ + 1];
+  int rstep[NMAX], prow[NMAX];   // the step that chose a row (-1: none yet), the row of a step
+  int bad, go;
+};
+
+// One chunk's steps in helper wave 0: x[m] the values of row lane + 64 m, on[m] all
+// bits while the row can be chosen, else 0.
+template <int RL>
+__device__ __forceinline__ void chunk_inverse(float (&x)[RL][16], int (&on)[RL], int k0, bool spd, int lane,
+                                              int& mine, bool& fine) {
+  float sc[RL];   // the factor of a pivot row of this chunk
+#pragma unroll
+  for (int m = 0; m < RL; ++m) sc[m] = 1.0f;
+#pragma unroll
+  for (int kq = 0; kq < 16; ++kq) {
+    float pr[16];
+    int p = 0;
+    auto take = [&](auto place, int pl) __attribute__((always_inline)) {
+      constexpr int m = decltype(place)::value;
+      if constexpr (m < RL) {
+        p = pl + 64 * m;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) pr[c] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x[m][c]), pl));
+      }
+    };
+    int pl = (k0 + kq) & 63, pm = (k0 + kq) >> 6;
+    if (!spd) {
+      // rank: the bits of |a|, then those of -2.0 for NaN, the lowest for a row already chosen
+      int f[RL], fl = INT32_MIN;
+#pragma unroll
+      for (int m = 0; m < RL; ++m) {
+        f[m] = min(__float_as_int(fmaxf(fabsf(x[m][kq]), -2.0f)), on[m] ^ INT32_MIN);
+        fl = max(fl, f[m]);
+      }
+      const int fm = imax_all(fl);
+      uint64_t hit = 0;   // lowest row of that rank
+#pragma unroll
+      for (int m = RL - 1; m >= 0; --m) {
+        const uint64_t h = __ballot(f[m] == fm);
+        pm = h ? m : pm;
+        hit = h ? h : hit;
+      }
+      pl = hit ? (int)__builtin_ctzll(hit) : 0;
+    }
+    if (pm < 2) {
+      if (pm == 0) take(std::integral_constant<int, 0>{}, pl);
+      else take(std::integral_constant<int, 1>{}, pl);
+    } else {
+      if (pm == 2) take(std::integral_constant<int, 2>{}, pl);
+      else take(std::integral_constant<int, 3>{}, pl);
+    }
+    const float pv = pr[kq];
+    fine = fine && pv != 0.0f && pv == pv;
+    mine = lane == kq ? p : mine;   // lane q keeps step q's row
+    const float rp = 1.0f / pv;
+    float l[RL];
+#pragma unroll
+    for (int m = 0; m < RL; ++m) {
+      const bool sel = lane + 64 * m == p;
+      const float f = x[m][kq] * rp;
+      l[m] = sel ? 0.0f : f;
+      x[m][kq] = sel ? 1.0f : -f;
+      sc[m] = sel ? rp : sc[m];
+      on[m] = sel ? 0 : on[m];
+    }
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+      if (c != kq) {
+#pragma unroll
+        for (int m = 0; m < RL; ++m) x[m][c] -= l[m] * pr[c];
+      }
+  }
+#pragma unroll
+  for (int m = 0; m < RL; ++m)
+#pragma unroll
+    for (int c = 0; c < 16; ++c) x[m][c] *= sc[m];
+}
+
+template <int ND>
+__global__ void __launch_bounds__((ND + ND / 2) * 64, ND == 8 ? 3 : 4) batched_tile_kernel(BatchArgs g) {
+  typedef float f32x16 __attribute__((ext_vector_type(16)));
+  typedef TileShared<ND> Sh;
+  constexpr int NMAX = Sh::NMAX, CW = Sh::CW, CS = Sh::CS, NH = Sh::NH, RL = NMAX / 64;
+  __shared__ __align__(16) Sh sh;
+  const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6);
+  // waves go to the four SIMDs in turn: wave 0, with the steps' chain, shares its
+  // SIMD with helper waves only
+  const bool holds = wid % 4 != 0 && wid != 11;
+  const int wv = holds ? wid - wid / 4 - 1 : (wid == 11 ? 3 : wid / 4);
+  const int li = lane & 31, hk = lane >> 5;
+  const int sid = g.list[blockIdx.x];   // (larger systems come first)
+  const SysDesc d = g.sys[sid];
+  const int n = d.n, nch = (n + CW - 1) / CW;
+  const int groups = (d.nrhs + BQ - 1) / BQ;
+
+  // The two kinds of waves take separate paths with the same barriers, so that
+  // neither carries the other's registers.
+  if (!holds) {
+    const int u = 64 * wv + lane;   // this thread's row
+    sh.rstep[u] = -1;
+    if (u == 0) sh.bad = 0;
+    for (int j = 0; j < ND; ++j) {   // (the accumulator waves stage A)
+      __syncthreads();
+      __syncthreads();
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int ch = 0; ch < nch; ++ch) {
+      const int k0 = CW * ch;
+      if (wv == 0) {
+        __builtin_amdgcn_s_setprio(3);
+        float* const cc = sh.chunk[ch & 1];
+        float x[RL][CW];
+        int on[RL], mine = 0;
+        bool fine = true;
+#pragma unroll
+        for (int m = 0; m < RL; ++m) {
+          const int row = lane + 64 * m;
+#pragma unroll
+          for (int q = 0; q < CW / 4; ++q) {
+            const float4 v = *reinterpret_cast<const float4*>(&cc[row * CS + 4 * q]);
+            x[m][4 * q] = v.x;
+            x[m][4 * q + 1] = v.y;
+            x[m][4 * q + 2] = v.z;
+            x[m][4 * q + 3] = v.w;
+          }
+          on[m] = row < CW * nch && sh.rstep[row] < 0 ? -1 : 0;
+        }
+        chunk_inverse<RL>(x, on, k0, d.spd != 0, lane, mine, fine);
+#pragma unroll
+        for (int m = 0; m < RL; ++m)
+#pragma unroll
+          for (int q = 0; q < CW / 4; ++q)
+            *reinterpret_cast<float4*>(&cc[(lane + 64 * m) * CS + 4 * q]) =
+                make_float4(x[m][4 * q], x[m][4 * q + 1], x[m][4 * q + 2], x[m][4 * q + 3]);
+        if (lane < CW) {
+          sh.prow[k0 + lane] = mine;
+          sh.rstep[mine] = k0 + lane;
+        }
+        if (lane == 0 && !fine) sh.bad = 1;
+        __builtin_amdgcn_s_setprio(0);
+      }
+      __syncthreads();   // B1: G is there, the last chunk's product is done
+      __syncthreads();   // B2: U is there
+      __syncthreads();   // B3: the next chunk is there
+    }
+    // ---- refinement
+    int worst = sh.bad ? -1 : 0;
+    const int pu = u < n ? sh.prow[u] : 0;   // (a row also when the system is bad: every step chose one)
+    double anorm = 0.0;
+#pragma unroll 1
+    for (int gq = 0; gq < groups && worst >= 0; ++gq) {
+      const int q0 = gq * BQ, nq = min(BQ, d.nrhs - q0);
+      const double* const b = d.b + (int64_t)q0 * n;
+      double x[BQ], prev[BQ];
+      int it[BQ];
+      bool act[BQ];
+#pragma unroll
+      for (int q = 0; q < BQ; ++q) {
+        x[q] = 0.0;
+        sh.rv[q][u] = q < nq && u < n ? b[(int64_t)q * n + u] : 0.0;
+        prev[q] = INFINITY;
+        it[q] = 0;
+        act[q] = q < nq;
+      }
+      __syncthreads();   // R0
+      for (;;) {
+#pragma unroll
+        for (int q = 0; q < BQ; ++q) sh.cv[q][u] = u < n ? (float)sh.rv[q][pu] : 0.0f;
+        __syncthreads();   // R1
+        __syncthreads();   // R2: yv
+#pragma unroll
+        for (int q = 0; q < BQ; ++q) {
+          if (act[q] && u < n) x[q] += (double)sh.yv[q][pu];
+          sh.xv[u][q] = x[q];
+        }
+        __syncthreads();   // R3
+        // r = b - A x and the row sums of |A|, one row per thread, columns in order
+        double acc[BQ], asum = 0.0;
+#pragma unroll
+        for (int q = 0; q < BQ; ++q) acc[q] = q < nq && u < n ? b[(int64_t)q * n + u] : 0.0;
+        if (u < n) {
+          const double* pa = d.a + u;
+          auto one = [&](double v, int j) __attribute__((always_inline)) {
+            const double2 x01 = *reinterpret_cast<const double2*>(&sh.xv[j][0]);
+            const double2 x23 = *reinterpret_cast<const double2*>(&sh.xv[j][2]);
+            acc[0] -= v * x01.x;
+            acc[1] -= v * x01.y;
+            acc[2] -= v * x23.x;
+            acc[3] -= v * x23.y;
+            asum += fabs(v);
+          };
+          int j = 0;
+          for (; j + 16 <= n; j += 16) {
+            double v[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) v[e] = pa[(int64_t)(j + e) * n];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) one(v[e], j + e);
+          }
+          for (; j < n; ++j) one(pa[(int64_t)j * n], j);
+        }
+        double mx[2 * BQ + 1];
+#pragma unroll
+        for (int q = 0; q < BQ; ++q) {
+          sh.rv[q][u] = acc[q];
+          mx[q] = fabs(acc[q]);
+          mx[BQ + q] = fabs(x[q]);
+        }
+        mx[2 * BQ] = asum;
+#pragma unroll
+        for (int e = 0; e < 2 * BQ + 1; ++e) {
+          for (int off = 32; off > 0; off >>= 1) mx[e] = fmax(mx[e], __shfl_xor(mx[e], off));
+          if (lane == 0) sh.red[wv][e] = mx[e];
+        }
+        __syncthreads();   // R4
+#pragma unroll
+        for (int e = 0; e < 2 * BQ + 1; ++e) {
+          mx[e] = sh.red[0][e];
+#pragma unroll
+          for (int w = 1; w < NH; ++w) mx[e] = fmax(mx[e], sh.red[w][e]);
+        }
+        if (anorm == 0.0) anorm = mx[2 * BQ];
+        bool go = false;
+#pragma unroll
+        for (int q = 0; q < BQ; ++q) {
+          if (!act[q]) continue;
+          ++it[q];
+          const double be = mx[q] / (anorm * mx[BQ + q] * (double)n * 0x1p-53);
+          if (be <= g.tol) {
+            act[q] = false;
+          } else if (!(be == be) || it[q] >= g.max_iter || (it[q] >= 2 && be > 0.5 * prev[q])) {
+            it[q] = -1;
+            act[q] = false;
+          } else {
+            prev[q] = be;
+            go = true;
+          }
+        }
+        if (u == 0) sh.go = go;
+        __syncthreads();   // R5
+        if (!go) break;
+      }
+#pragma unroll
+      for (int q = 0; q < BQ; ++q) {
+        if (q >= nq || worst < 0) continue;   // (nothing is written after a right-hand side that failed)
+        if (u < n) d.x[(int64_t)(q0 + q) * n + u] = x[q];
+        worst = it[q] < 0 ? -1 : max(worst, it[q]);
+      }
+      if (u == 0) sh.go = worst >= 0;
+      __syncthreads();   // R6
+    }
+    if (u == 0) g.status[sid] = worst;
+    return;
+  }
+
+  const int row0 = 32 * wv + 4 * hk;   // element r of a tile: row row0 + 8 (r / 4) + r % 4, column li
+  const int nj = (n + 31) / 32;        // tiles of a row (and accumulator waves) in use
+  f32x16 a[ND];
+  // A is column-major and a lane of a tile holds columns: tile by tile through LDS
+  // (consecutive threads read consecutive rows), the next tile's reads in flight
+  {
+    constexpr int TS = NMAX + 4, PT = NMAX * 32 / (ND * 64);   // column stride, elements of a thread
+    static_assert(32 * TS <= 2 * NMAX * CS, "a tile column fits the chunk buffers");
+    float* const st = sh.chunk[0];
+    const int th = 64 * wv + lane, sr = th % NMAX, sc = th / NMAX;   // row, first column (then + 2)
+    double v[PT];
+    auto fetch = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < PT; ++e) {
+        const int c = 32 * j + sc + 2 * e;
+        const double w = d.a[min(sr, n - 1) + (int64_t)min(c, n - 1) * n];
+        v[e] = sr < n && c < n ? w : (sr == c && c < CW * nch ? 1.0 : 0.0);   // the rest of the last chunk: identity
+      }
+    };
+    fetch(0);
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+#pragma unroll
+      for (int e = 0; e < PT; ++e) st[(sc + 2 * e) * TS + sr] = (float)v[e];
+      if (j + 1 < nj) fetch(j + 1);
+      else {
+#pragma unroll
+        for (int e = 0; e < PT; ++e) v[e] = 0.0;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 w = *reinterpret_cast<const float4*>(&st[li * TS + row0 + 8 * q]);
+        a[j][4 * q] = w.x;
+        a[j][4 * q + 1] = w.y;
+        a[j][4 * q + 2] = w.z;
+        a[j][4 * q + 3] = w.w;
+      }
+      __syncthreads();
+    }
+  }
+  if (li < CW) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sh.chunk[0][(row0 + 8 * (r >> 2) + (r & 3)) * CS + li] = a[0][r];
+  }
+  __syncthreads();
+  int hits = 0;
+  auto drop = [&](f32x16& v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = hits & (1 << r) ? 0.0f : v[r];
+  };
+#pragma unroll 1
+  for (int ch = 0;; ++ch) {
+    const int k0 = CW * ch, h = ch & 1;
+    const float* const cc = sh.chunk[h];
+    if (ch > 0) {
+      // ---- the last chunk's G U in the tiles but this chunk's, then its own
+      // columns back into their tile
+      const float* const cp = sh.chunk[h ^ 1];
+      const int skip = ch < nch ? ch >> 1 : ND;
+      if (wv < nj) {
+        float l[CW / 2];
+#pragma unroll
+        for (int s = 0; s < CW / 2; ++s) l[s] = cp[(32 * wv + li) * CS + 2 * s + hk];
+#pragma unroll
+        for (int j = 0; j < ND; ++j)
+          if (j < nj && j != skip) {
+            drop(a[j]);
+#pragma unroll
+            for (int s = 0; s < CW / 2; ++s)
+              a[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(l[s], sh.ubuf[(2 * s + hk) * NMAX + 32 * j + li], a[j], 0, 0, 0);
+          }
+#pragma unroll
+        for (int j = 0; j < ND; ++j)
+          if (j == (ch - 1) >> 1 && (li / CW) != h) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) a[j][r] = cp[(row0 + 8 * (r >> 2) + (r & 3)) * CS + li % CW];
+          }
+      }
+      if (ch == nch) break;
+    }
+    __syncthreads();   // B1
+    // ---- the chunk's pivot rows to ubuf; they count as zero from here (bit r of
+    // `hits`: element r's row is one)
+    hits = 0;
+    if (wv < nj) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int4 v = *reinterpret_cast<const int4*>(&sh.rstep[row0 + 8 * q]);
+        const int rs[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int st = rs[e] - k0;
+          hits |= st >= 0 ? 1 << (4 * q + e) : 0;
+          if (st >= 0) {
+#pragma unroll
+            for (int j = 0; j < ND; ++j) sh.ubuf[st * NMAX + 32 * j + li] = a[j][4 * q + e];
+          }
+        }
+      }
+    }
+    __syncthreads();   // B2
+    if (ch + 1 < nch && wv < nj) {
+      // ---- the tile with the next chunk, and the chunk out to LDS
+      const int jn = (ch + 1) >> 1;
+      float l[CW / 2];
+#pragma unroll
+      for (int s = 0; s < CW / 2; ++s) l[s] = cc[(32 * wv + li) * CS + 2 * s + hk];
+#pragma unroll
+      for (int j = 0; j < ND; ++j)
+        if (j == jn) {
+          drop(a[j]);
+#pragma unroll
+          for (int s = 0; s < CW / 2; ++s)
+            a[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(l[s], sh.ubuf[(2 * s + hk) * NMAX + 32 * j + li], a[j], 0, 0, 0);
+        }
+      float* const cn = sh.chunk[h ^ 1];
+#pragma unroll
+      for (int j = 0; j < ND; ++j)
+        if (j == jn && (li / CW) != h) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) cn[(row0 + 8 * (r >> 2) + (r & 3)) * CS + li % CW] = a[j][r];
+        }
+    }
+    __syncthreads();   // B3
+  }
+  // ---- refinement: y = M c, row sums over the half wave's 32 columns and the tiles
+  int ok = !sh.bad;
+#pragma unroll 1
+  for (int gq = 0; gq < groups && ok; ++gq) {
+    const int nq = min(BQ, d.nrhs - gq * BQ);
+    __syncthreads();   // R0
+    for (;;) {
+      __syncthreads();   // R1
+      if (wv < nj) {
+#pragma unroll 1
+        for (int q = 0; q < nq; ++q) {
+          float v[16];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) v[r] = 0.0f;
+#pragma unroll
+          for (int j = 0; j < ND; ++j)
+            if (j < nj) {
+              const float c = sh.cv[q][32 * j + li];
+#pragma unroll
+              for (int r = 0; r < 16; ++r) v[r] = fmaf(a[j][r], c, v[r]);
+            }
+          // halves of the values change hands until lane li has row (li >> 1) & 15's sum
+#pragma unroll
+          for (int w = 8; w >= 1; w >>= 1) {
+            const bool up = (li & (2 * w)) != 0;
+#pragma unroll
+            for (int r = 0; r < w; ++r) {
+              const float keep = up ? v[r + w] : v[r], send = up ? v[r] : v[r + w];
+              v[r] = keep + __shfl_xor(send, 2 * w);
+            }
+          }
+          const float y = v[0] + __shfl_xor(v[0], 1);
+          const int r = li >> 1;
+          if ((li & 1) == 0) sh.yv[q][row0 + 8 * (r >> 2) + (r & 3)] = y;
+        }
+      }
+      __syncthreads();   // R2
+      __syncthreads();   // R3
+      __syncthreads();   // R4
+      __syncthreads();   // R5
+      if (!sh.go) break;
+    }
+    __syncthreads();   // R6
+    ok = sh.go;
+  }
+}
+
 __global__ void reset_counters_kernel(int* c, int k) {
   if ((int)threadIdx.x < k) c[threadIdx.x] = 0;
 }
 
 // ---- variants and buckets -------------------------------------------------------------
 struct Variant {
-  int ty, tx, ri, rj;   // thread grid TY x TX, RI x RJ values per thread
+  int ty, tx, ri, rj;   // thread grid TY x TX, RI x RJ values per thread (tiles: 32 rows, RI tiles each way)
   void (*kernel)(BatchArgs);
+  int nt;               // threads
+  bool queue;           // persistent workgroups on the bucket's work queue
 };
 const Variant kVariants[] = {
-    {8, 8, 4, 4, batched_solve_kernel<8, 8, 4, 4>},        // n <= 32, one wave
-    {8, 8, 8, 8, batched_solve_kernel<8, 8, 8, 8>},        // n <= 64, one wave
-    {16, 16, 4, 4, batched_solve_kernel<16, 16, 4, 4>},    // n <= 64, four waves
-    {16, 16, 8, 8, batched_solve_kernel<16, 16, 8, 8>},    // n <= 128
-    {32, 32, 4, 4, batched_solve_kernel<32, 32, 4, 4>},    // n <= 128, sixteen waves
-    {32, 32, 8, 8, batched_solve_kernel<32, 32, 8, 8>},    // n <= 256, sixteen waves (register spills)
-    {16, 32, 16, 8, batched_solve_kernel<16, 32, 16, 8>},  // n <= 256, eight waves
+    {8, 8, 4, 4, batched_solve_kernel<8, 8, 4, 4>, 64, true},        // n <= 32, one wave
+    {8, 8, 8, 8, batched_solve_kernel<8, 8, 8, 8>, 64, true},        // n <= 64, one wave
+    {16, 16, 4, 4, batched_solve_kernel<16, 16, 4, 4>, 256, true},    // n <= 64, four waves
+    {32, 12, 4, 4, batched_tile_kernel<4>, 384, false},           // n <= 128, accumulator tiles
+    {32, 24, 8, 8, batched_tile_kernel<8>, 768, false},           // n <= 256, accumulator tiles
 };
 constexpr int kBuckets = 4;
 const int kBucketMax[kBuckets] = {32, 64, 128, 256};
-const std::vector<int> kCandidates[kBuckets] = {{0, 1, 2}, {1, 2}, {3, 4}, {6, 5}};
+const std::vector<int> kCandidates[kBuckets] = {{0, 1, 2}, {1, 2}, {3}, {4}};
 
 }  // namespace
 
@@ -342,15 +817,17 @@ namespace {
 
 unsigned resident_grid(int v) {
   int per_cu = 0;
-  const int nt = kVariants[v].ty * kVariants[v].tx;
+  const int nt = kVariants[v].nt;
   ZH_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kVariants[v].kernel),
                                                         nt, 0));
   return (unsigned)(std::max(per_cu, 1) * device_cu_count());
 }
 
 void launch_bucket(const BatchPlan& P, int b, int v, hipStream_t s) {
-  const int nt = kVariants[v].ty * kVariants[v].tx;
-  const unsigned grid = std::min<unsigned>(P.grid[b], (unsigned)std::max(1, P.bucket_count[b]));
+  const int nt = kVariants[v].nt;
+  // (the tile kernels take one system per workgroup, in list order)
+  const unsigned grid = kVariants[v].queue ? std::min<unsigned>(P.grid[b], (unsigned)std::max(1, P.bucket_count[b]))
+                                           : (unsigned)P.bucket_count[b];
   BatchArgs args = P.args[b];
   void* kargs[] = {&args};
   ZH_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(kVariants[v].kernel), dim3(grid), dim3(nt), kargs, 0, s));
