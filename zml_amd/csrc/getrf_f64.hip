@@ -129,7 +129,10 @@ int32_t* perm_pairs_buffer(int slot) {
 int32_t* compose_perm(int k1, int k2, const int32_t* ipiv, hipStream_t s, int slot) {
   if (k2 - k1 + 1 > panel::PERM_MAX / 2) throw std::runtime_error("compose_perm: block too wide");
   int32_t* pairs = perm_pairs_buffer(slot);
-  hipLaunchKernelGGL(panel::compose_perm_kernel, dim3(1), dim3(64), 0, s, k1, k2, ipiv, pairs);
+  if (k2 - k1 < 256)
+    hipLaunchKernelGGL(panel::compose_perm_kernel<256>, dim3(1), dim3(512), 0, s, k1, k2, ipiv, pairs);
+  else
+    hipLaunchKernelGGL(panel::compose_perm_kernel<512>, dim3(1), dim3(1024), 0, s, k1, k2, ipiv, pairs);
   ZH_LAUNCH_CHECK();
   return pairs;
 }

@@ -22,6 +22,7 @@
 #pragma once
 
 #include "zmlhip_internal.hpp"
+#include "perm.hpp"
 
 namespace zmlhip {
 namespace panel {
@@ -383,90 +384,28 @@ leaf_kernel(int64_t M, int Wn, T* __restrict__ P, int64_t ld, int32_t* __restric
 // ---- row interchanges through the composed permutation ----------------------
 constexpr int PERM_MAX = 1024;  // pairs (2 x block of 512 interchanges)
 
-// Composes the interchanges i <-> ipiv[i]-1 for i = k1..k2 (ascending, every
-// ipiv[i]-1 >= i) into a list of moves dst <- src over the rows touched.
-// One wave: the rows beyond the block enter an open-addressing table
-// (row -> slot) in parallel, each interchange's partner slot is looked up in
-// parallel, one lane then walks the interchanges in order (a swap of two LDS
-// words each), and the slots whose content changed become moves, compacted by
-// a ballot. pairs[0] = count, then (dst, src) pairs in slot order.
-constexpr int PERM_HT = 2 * PERM_MAX;   // power of two, load factor <= 1/4
-static_assert((PERM_HT & (PERM_HT - 1)) == 0, "table size must be a power of two");
-__device__ __forceinline__ uint32_t perm_hash(int p) { return ((uint32_t)p * 2654435761u) & (PERM_HT - 1); }
-__global__ void __launch_bounds__(64)
+// Composes the interchanges i <-> ipiv[i]-1 for i = k1..k2 (ascending, at most NS of
+// them) into a list of moves dst <- src over the rows touched: pairs[0] = count, then
+// (dst, src) pairs. One workgroup of 2 NS threads: 512 interchanges
+// 25 us, 200 10 us; one lane walking them took 52 and 23 us.
+template <int NS>
+__global__ void __launch_bounds__(2 * NS)
 compose_perm_kernel(int k1, int k2, const int32_t* __restrict__ ipiv, int32_t* __restrict__ pairs) {
-  __shared__ int32_t pos[PERM_MAX], cont[PERM_MAX], partner[PERM_MAX / 2];
-  __shared__ int32_t hkey[PERM_HT], hslot[PERM_HT];
+  __shared__ __align__(16) int2 ev[NS];
+  __shared__ int node[2 * NS];
   __shared__ int s_n;
-  const int lane = threadIdx.x;
-  const int kb = k2 - k1 + 1;
-  for (int q = lane; q < kb; q += 64) { pos[q] = k1 + q; cont[q] = k1 + q; }
-  for (int q = lane; q < PERM_HT; q += 64) hkey[q] = -1;
-  if (lane == 0) s_n = kb;
+  const int t = threadIdx.x, cnt = k2 - k1 + 1;
+  if (t == 0) s_n = 0;
+  if (t < NS) ev[t] = t < cnt ? make_int2(k1 + t, ipiv[k1 + t] - 1) : make_int2(-1, -1);
   __syncthreads();
-  // the distinct rows beyond the block enter the table
-  for (int q = lane; q < kb; q += 64) {
-    const int p = ipiv[k1 + q] - 1;
-    if (p > k2) {
-      uint32_t h = perm_hash(p);
-      for (;;) {
-        const int prev = atomicCAS(&hkey[h], -1, p);
-        if (prev == -1 || prev == p) break;
-        h = (h + 1) & (PERM_HT - 1);
-      }
-    }
+  int dst, src;
+  if (compose_swaps<NS>(ev, cnt, node, dst, src) && dst != src) {
+    const int at = atomicAdd(&s_n, 1);
+    pairs[1 + 2 * at] = dst;
+    pairs[2 + 2 * at] = src;
   }
   __syncthreads();
-  // each of them gets a slot after the block's
-  for (int h = lane; h < PERM_HT; h += 64) {
-    const int key = hkey[h];
-    if (key >= 0) {
-      const int sl = atomicAdd(&s_n, 1);
-      hslot[h] = sl;
-      pos[sl] = key;
-      cont[sl] = key;
-    }
-  }
-  __syncthreads();
-  // the slot each interchange swaps with
-  for (int q = lane; q < kb; q += 64) {
-    const int p = ipiv[k1 + q] - 1;
-    int qp;
-    if (p <= k2) {
-      qp = p - k1;
-    } else {
-      uint32_t h = perm_hash(p);
-      while (hkey[h] != p) h = (h + 1) & (PERM_HT - 1);
-      qp = hslot[h];
-    }
-    partner[q] = qp;
-  }
-  __syncthreads();
-  if (lane == 0) {
-    for (int q = 0; q < kb; ++q) {
-      const int qp = partner[q];
-      if (qp != q) {
-        const int tmp = cont[q];
-        cont[q] = cont[qp];
-        cont[qp] = tmp;
-      }
-    }
-  }
-  __syncthreads();
-  const int n = s_n;
-  int c = 0;
-  for (int q0 = 0; q0 < n; q0 += 64) {
-    const int q = q0 + lane;
-    const bool moved = q < n && cont[q] != pos[q];
-    const uint64_t m = __ballot(moved);
-    if (moved) {
-      const int at = c + (int)__popcll(m & ((1ull << lane) - 1ull));
-      pairs[1 + 2 * at] = pos[q];
-      pairs[2 + 2 * at] = cont[q];
-    }
-    c += (int)__popcll(m);
-  }
-  if (lane == 0) pairs[0] = c;
+  if (t == 0) pairs[0] = s_n;
 }
 
 // Applies the moves to columns [0, ncols) of a row-major matrix: every
