@@ -5,6 +5,7 @@
 #include "zmlhip_internal.hpp"
 
 #include <algorithm>
+#include <exception>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -78,20 +79,21 @@ size_t vspan(int64_t n, int64_t inc) {
   return (size_t)((n - 1) * (inc < 0 ? -inc : inc) + 1);
 }
 
-// Device copy of a host buffer, freed on scope exit.
+// Device copy of a host buffer, given back on scope exit (a call that ends in an
+// error may have work of its other streams in flight: its blocks are freed, which
+// waits for the device).
 struct DevBuf {
   void* p = nullptr;
-  size_t bytes = 0;
+  size_t bytes = 0, got = 0;
+  const int unwinding = std::uncaught_exceptions();
   DevBuf() = default;
   explicit DevBuf(size_t b) : bytes(b) {
-    if (b) ZH_CHECK(hipMalloc(&p, b));
+    if (b) p = host_block(b, &got);
   }
   DevBuf(const void* host, size_t b, hipStream_t s) : DevBuf(b) {
     if (b && host) ZH_CHECK(hipMemcpyAsync(p, host, b, hipMemcpyHostToDevice, s));
   }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
+  ~DevBuf() { host_block_done(p, got, std::uncaught_exceptions() == unwinding); }
   void to_host(void* host, hipStream_t s) const {
     if (bytes && host) ZH_CHECK(hipMemcpyAsync(host, p, bytes, hipMemcpyDeviceToHost, s));
   }

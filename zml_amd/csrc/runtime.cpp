@@ -29,6 +29,7 @@ struct DeviceState {
   int reserved_cus[kSparing] = {};
   hipStream_t reserved[kSparing] = {};   // every CU but the first reserved_cus[i]
   hipEvent_t ev[kEvents] = {};
+  std::vector<Buf> kept;        // idle device blocks of the host-memory calls
   hipEvent_t fence = nullptr;   // end of the previous call of this thread on this device
   bool fence_set = false;
 };
@@ -41,6 +42,7 @@ struct ThreadState {
       if (hipSetDevice(kv.first) != hipSuccess) continue;
       for (auto& b : kv.second.slot)
         if (b.ptr) (void)hipFree(b.ptr);
+      for (auto& b : kv.second.kept) (void)hipFree(b.ptr);
       if (kv.second.stream) (void)hipStreamDestroy(kv.second.stream);
       for (auto& st : kv.second.aux)
         if (st) (void)hipStreamDestroy(st);
@@ -133,6 +135,55 @@ void* workspace(size_t bytes, int slot) {
     b.bytes = sz;
   }
   return b.ptr;
+}
+
+// A call on host memory takes two to four blocks; allocating and freeing them cost
+// 65 of the 555 us of a 200 x 200 solve (a free waits for the device). Blocks of up to
+// 16 MiB are kept, at most eight per thread and device: above that a call's copies
+// take milliseconds and the allocation no longer shows.
+constexpr size_t kKeptBlock = size_t(16) << 20;
+constexpr size_t kKeptBlocks = 8;
+
+void* host_block(size_t bytes, size_t* got) {
+  std::vector<Buf>& kept = current().kept;
+  size_t best = kept.size();
+  for (size_t i = 0; i < kept.size(); ++i)
+    if (kept[i].bytes >= bytes && (best == kept.size() || kept[i].bytes < kept[best].bytes)) best = i;
+  if (best < kept.size()) {
+    const Buf b = kept[best];
+    kept.erase(kept.begin() + (std::ptrdiff_t)best);
+    *got = b.bytes;
+    return b.ptr;
+  }
+  void* p = nullptr;
+  *got = bytes <= kKeptBlock ? align_up(bytes, 1 << 16) : bytes;
+  hipError_t e = hipMalloc(&p, *got);
+  if (e == hipErrorOutOfMemory && !kept.empty()) {
+    (void)hipGetLastError();
+    for (auto& b : kept) (void)hipFree(b.ptr);
+    kept.clear();
+    e = hipMalloc(&p, *got);
+  }
+  ZH_CHECK(e);
+  return p;
+}
+
+void host_block_done(void* p, size_t got, bool keep) noexcept {
+  if (!p) return;
+  if (keep && got <= kKeptBlock) {
+    try {
+      std::vector<Buf>& kept = current().kept;
+      if (kept.size() < kKeptBlocks) {
+        Buf b;
+        b.ptr = p;
+        b.bytes = got;
+        kept.push_back(b);
+        return;
+      }
+    } catch (...) {
+    }
+  }
+  (void)hipFree(p);
 }
 
 hipStream_t host_api_stream() {

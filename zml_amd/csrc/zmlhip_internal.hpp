@@ -87,6 +87,11 @@ void* workspace(size_t bytes, int slot = 0);
 
 // Stream used by the synchronous host-pointer entry points of this thread.
 hipStream_t host_api_stream();
+// Device memory of a call on host memory, from this thread's kept blocks or new; *got
+// is its size. Its work must be ordered on host_api_stream(). host_block_done gives it
+// back: kept for this thread's next such call when `keep` and small, else freed.
+void* host_block(size_t bytes, size_t* got);
+void host_block_done(void* p, size_t got, bool keep) noexcept;
 
 // Internal streams (default priority) and timing-free events of this thread
 // on the current device, used to overlap panel factorization with updates.
