@@ -127,10 +127,11 @@ int zmlhip_set_panel_spin_limit(long polls);
  * MI355X); a negative value restores it, 0 makes every block column take the
  * one-launch panel. Process-wide. No counterpart in the reference. */
 int zmlhip_set_panel_one_launch_rows(long rows);
-/* FP64 GEMMs (zmlhip_dgemm and the GEMMs inside the FP64 factorizations)
+/* GEMMs (zmlhip_dgemm, zmlhip_sgemm and the GEMMs inside the factorizations)
  * whose shapes allow it move their operand slabs from global memory to LDS
- * with the load unit (on = 1, the default); on = 0 makes every FP64 GEMM stage
- * them through registers. The two kernels give the same results bit for bit.
+ * with the load unit (on = 1, the default); on = 0 makes every GEMM stage them
+ * through registers. For zmlhip_dgemm, zmlhip_sgemm and the FP64 factorizations
+ * the two kernels give the same results bit for bit.
  * Returns the previous setting. Process-wide. No counterpart in the reference. */
 int zmlhip_set_gemm_lds_dma(int on);
 /* LU leaves of more than one workgroup publish column k + 1's pivot candidates
@@ -221,8 +222,8 @@ int zmlhip_batch_plan_create(zmlhip_batch_plan **plan, int count, const int *n, 
                              double *const *x, const zmlhip_ir_opts *opts, int autotune, void *stream);
 int zmlhip_batch_plan_execute(zmlhip_batch_plan *plan, void *stream);
 int zmlhip_batch_plan_status(zmlhip_batch_plan *plan, int *status, void *stream);
-/* thread rows of the grid, matrix rows per thread (their product bounds the
- * bucket's n) and system count of the 4 size buckets (n <= 32, 64, 128, 256) */
+/* thread rows of the grid, matrix rows per thread (n <= 32, 64) or rows of an
+ * accumulator tile, tiles (n <= 128, 256) (their product bounds the bucket's n) and system count of the 4 size buckets (n <= 32, 64, 128, 256) */
 int zmlhip_batch_plan_shapes(const zmlhip_batch_plan *plan, int *tg, int *r, int *count);
 int zmlhip_batch_plan_destroy(zmlhip_batch_plan *plan);
 
