@@ -341,7 +341,8 @@ struct TileShared {
   double xv[NMAX][BQ], rv[BQ][NMAX];
   double red[NH][2 * BQ + 1];
   int rstep[NMAX], prow[NMAX];   // the step that chose a row (-1: none yet), the row of a step
-  int bad, go;
+  int bad;
+  int again, solved;   // another step of this group (written before R5); the group did not fail (before R6)
 };
 
 // One chunk's steps in helper wave 0: x[m] the values of row lane + 64 m, on[m] all
@@ -578,7 +579,7 @@ __global__ void __launch_bounds__((ND + ND / 2) * 64, ND == 8 ? 3 : 4) batched_t
             go = true;
           }
         }
-        if (u == 0) sh.go = go;
+        if (u == 0) sh.again = go;
         __syncthreads();   // R5
         if (!go) break;
       }
@@ -588,7 +589,7 @@ __global__ void __launch_bounds__((ND + ND / 2) * 64, ND == 8 ? 3 : 4) batched_t
         if (u < n) d.x[(int64_t)(q0 + q) * n + u] = x[q];
         worst = it[q] < 0 ? -1 : max(worst, it[q]);
       }
-      if (u == 0) sh.go = worst >= 0;
+      if (u == 0) sh.solved = worst >= 0;   // (a word of its own: a late wave may still be reading `again`)
       __syncthreads();   // R6
     }
     if (u == 0) g.status[sid] = worst;
@@ -761,10 +762,10 @@ __global__ void __launch_bounds__((ND + ND / 2) * 64, ND == 8 ? 3 : 4) batched_t
       __syncthreads();   // R3
       __syncthreads();   // R4
       __syncthreads();   // R5
-      if (!sh.go) break;
+      if (!sh.again) break;
     }
     __syncthreads();   // R6
-    ok = sh.go;
+    ok = sh.solved;
   }
 }
 
