@@ -102,7 +102,8 @@ int zmlhip_dlange(int layout, char norm, int m, int n, const double *a, int lda,
                   void *stream);
 
 /* ---- LAPACK (device pointers; ipiv and info are device memory) -------- */
-/* LAPACKE_dlaswp (src/linalg/lapack.zig:375; lapack/laswp.zig:12-95) */
+/* LAPACKE_dlaswp (src/linalg/lapack.zig:375; lapack/laswp.zig:12-95). An entry of
+ * ipiv below 1 names no row: here and in zmlhip_dgetrs it makes no interchange. */
 int zmlhip_dlaswp(int layout, int n, double *a, int lda, int k1, int k2, const int *ipiv,
                   int incx, void *stream);
 /* LAPACKE_dgetrf (src/linalg/lapack.zig:1169; lapack/getrf.zig:14-152).

@@ -98,7 +98,7 @@ laswp_kernel(int64_t ncols, double* __restrict__ a, int64_t sr, int64_t sc, int 
   const int steps = inc > 0 ? k2 - k1 + 1 : k1 - k2 + 1;   // (k1..k2 stepping by inc)
   for (int s0 = 0; s0 < steps; s0 += LW_NS) {
     const int cnt = steps - s0 < LW_NS ? steps - s0 : LW_NS;
-    if (t < cnt) ev[t] = make_int2(k1 + inc * (s0 + t), ipiv[ix0 + (int64_t)(s0 + t) * incx] - 1);
+    if (t < cnt) ev[t] = swap_entry(k1 + inc * (s0 + t), ipiv[ix0 + (int64_t)(s0 + t) * incx]);
     else if (t < LW_NS) ev[t] = make_int2(-1, -1);
     __syncthreads();
     int dst, src;

@@ -396,7 +396,7 @@ compose_perm_kernel(int k1, int k2, const int32_t* __restrict__ ipiv, int32_t* _
   __shared__ int s_n;
   const int t = threadIdx.x, cnt = k2 - k1 + 1;
   if (t == 0) s_n = 0;
-  if (t < NS) ev[t] = t < cnt ? make_int2(k1 + t, ipiv[k1 + t] - 1) : make_int2(-1, -1);
+  if (t < NS) ev[t] = t < cnt ? swap_entry(k1 + t, ipiv[k1 + t]) : make_int2(-1, -1);
   __syncthreads();
   int dst, src;
   if (compose_swaps<NS>(ev, cnt, node, dst, src) && dst != src) {

@@ -6,8 +6,15 @@
 
 namespace zmlhip {
 
-// Where the interchanges ev[0], ev[1], .., ev[cnt - 1] (rows x <-> y, in this order;
-// in LDS, 16-byte aligned, cnt <= NS, entry cnt (-1, -1) when cnt is odd) leave every row they touch. 2 NS threads, two per interchange:
+// An interchange of row i with row ip - 1 as compose_swaps takes it. An entry of ipiv
+// below 1 names no row (a cleared ipiv): that interchange touches nothing.
+__device__ __forceinline__ int2 swap_entry(int i, int32_t ip) {
+  return i >= 0 && ip >= 1 ? make_int2(i, ip - 1) : make_int2(-1, -1);
+}
+
+// Where the interchanges ev[0], ev[1], .., ev[cnt - 1] (rows x <-> y, in this order,
+// each from swap_entry; in LDS, 16-byte aligned, cnt <= NS, entry cnt (-1, -1) when
+// cnt is odd) leave every row they touch. 2 NS threads, two per interchange:
 // thread 2 s + side stands for "the content of row ev[s].x (side 0) or ev[s].y after
 // interchange s", which is what the other row held before: the content after the last
 // earlier interchange that touched it, or its own row. Those links, found by a scan
@@ -23,10 +30,11 @@ template <int NS>
 __device__ __forceinline__ bool compose_swaps(const int2* ev, int cnt, int* node, int& dst, int& src) {
   const int t = threadIdx.x, s0 = t >> 1;
   const int w0 = __builtin_amdgcn_readfirstlane(s0 & ~31);   // the wave's first interchange
-  const bool mine = s0 < cnt;
-  const int2 me = mine ? ev[s0] : make_int2(-1, -2);
-  const int row = t & 1 ? me.y : me.x, other = t & 1 ? me.x : me.y;
-  int link = ~other;                           // < 0: the row itself
+  const int2 me = s0 < cnt ? ev[s0] : make_int2(-1, -1);
+  const bool mine = me.x >= 0;
+  // (-2 is in no entry: a thread without an interchange finds no link and is none's)
+  const int row = !mine ? -2 : t & 1 ? me.y : me.x, other = !mine ? -2 : t & 1 ? me.x : me.y;
+  int link = mine ? ~other : -1;               // < 0: the row itself
   bool later = false;                          // touched again
   // two entries per read (the list ends with an empty one when cnt is odd)
   const int4* const ev2 = reinterpret_cast<const int4*>(ev);
