@@ -51,7 +51,13 @@ int zmlhip_profile_collect(int kind, double *ms, long long *launches, double *fl
                            double *bytes);
 
 /* ---- BLAS (device pointers) ------------------------------------------- */
-/* cblas_dgemm (src/cblas.zig:526; blas/gemm.zig:14-1033) */
+/* cblas_dgemm (src/cblas.zig:526; blas/gemm.zig:14-1033). The matrix products
+ * queue their kernels and wait for nothing. A product too small to fill the CUs
+ * cuts a long k into parts whose sums are added in order; the parts follow from
+ * the shape alone, so a call recorded into a graph gives the same bits as a direct
+ * one. Their memory (32 MiB on 256 CUs) is allocated by a thread's first such call on
+ * a device and kept until the thread ends; recorded calls, and calls for which
+ * there is no memory, do without it. */
 int zmlhip_dgemm(int layout, int transa, int transb, int m, int n, int k, double alpha,
                  const double *a, int lda, const double *b, int ldb, double beta, double *c,
                  int ldc, void *stream);

@@ -15,8 +15,8 @@
 //    tiles whose operand slabs go from global memory to LDS by the load unit; 71
 //    TF/s FP64, 122 TF/s FP32 at 4096^3 on MI355X;
 //  - gemm_small_kernel (every shape, FP64 and FP32): 64 x 64 tiles staged through
-//    registers, four workgroups per CU, with k split over workgroups where even
-//    these are few.
+//    registers, four workgroups per CU, with k cut into parts that are summed on their
+//    own, one workgroup each, where even these are few.
 // A 256-thread workgroup's four waves each own a quarter of the tile. K advances in
 // slabs of 16 through double-buffered LDS. The MFMA is issued as C^T = op(B)^T
 // op(A)^T so that the 16 lanes of an output group hold 16 consecutive rows of one
@@ -91,14 +91,25 @@ __device__ __forceinline__ void tile_coords(int64_t bid, int64_t ntm, int64_t nt
 // FP64, 100 TF/s FP32 at 4096^3), by the number of tiles below about 2000^2.
 // Update form C <- C +- op(A) op(B) (beta 1, alpha +-1): the accumulators start
 // from C and B is staged negated for alpha -1, so the epilogue only stores.
-// part != nullptr: the K range is split over gridDim.y workgroups, each of which
-// leaves its plain sum in part + z m n (m x n, column-major) for splitk_sum_kernel.
+// PARTS: k in parts of kper, each summed on its own and then added to the sum of the
+// earlier ones. With part != nullptr gridDim.y workgroups take one part each and
+// leave its sum in part + z m n (m x n, column-major) for splitk_sum_kernel; without,
+// one workgroup goes through the parts of its tile itself: the same bits, for a call
+// that has no memory for them.
 // On MI355X, against 128 x 128 tiles: 1001 x 1500 x 777 143 -> 78 us, 1024^3 145 ->
 // 67 us, 124 x 918 x 5130 (k split 17 ways) 838 -> 43 us.
 constexpr int SM = 64, SLD = SM + 2;
 
-template <typename T, bool TA, bool TB>
-__global__ void __launch_bounds__(NT, 4)
+// The last rounding steps of a product whose sum is s.
+template <typename T>
+__device__ __forceinline__ T scaled_sum(T s, T alpha, T beta, T c) {
+#pragma clang fp contract(off)
+  const T v = alpha * s;
+  return beta == T(0) ? v : (beta == T(1) ? c + v : fma(beta, c, v));
+}
+
+template <typename T, bool TA, bool TB, bool PARTS>
+__global__ void __launch_bounds__(NT, PARTS ? 2 : 4)
 gemm_small_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict__ A, int64_t lda,
                   const T* __restrict__ B, int64_t ldb, T beta, T* __restrict__ C, int64_t ldc, int tri,
                   int64_t tri_tiles, int64_t kper, T* __restrict__ part) {
@@ -113,7 +124,8 @@ gemm_small_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict_
   if (tri == kUpper && col0 + SM - 1 < row0) return;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave & 1, wn = wave >> 1;
   const int lr = lane & 15, lk = lane >> 4;
-  const int64_t kb = blockIdx.y * kper, ke = kb + kper < k ? kb + kper : k;
+  const int64_t kb = PARTS ? blockIdx.y * kper : 0;
+  int64_t ke = PARTS && kb + kper < k ? kb + kper : k;
 
   // element q of this thread: (i, l) = (t & 63, (t >> 6) + 4 q) where the operand is
   // contiguous along m / n, ((t >> 4) + 16 q, t & 15) where it is along k
@@ -148,7 +160,7 @@ gemm_small_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict_
       }
     }
   };
-  const bool cinit = !part && beta == T(1) && (alpha == T(1) || alpha == T(-1));
+  const bool cinit = !PARTS && beta == T(1) && (alpha == T(1) || alpha == T(-1));
   const bool negb = cinit && alpha == T(-1);
   auto store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -176,12 +188,12 @@ gemm_small_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict_
           acc[x][y][r] = v;   // (outside C, or in the other triangle: computed, not stored)
         }
       }
-  if (kb < ke) {
-    load(kb);
+  auto sum = [&](int64_t k1) __attribute__((always_inline)) {   // k1 .. ke - 1 onto the accumulators
+    load(k1);
     store(0);
     __syncthreads();
     int cur = 0;
-    for (int64_t k0 = kb; k0 < ke; k0 += BK, cur ^= 1) {
+    for (int64_t k0 = k1; k0 < ke; k0 += BK, cur ^= 1) {
       const bool more = k0 + BK < ke;
       if (more) load(k0 + BK);
       const T* as = As[cur] + wm * 32 + lr;
@@ -201,6 +213,28 @@ gemm_small_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict_
       }
       if (more) store(cur ^ 1);
       __syncthreads();
+    }
+  };
+  if (kb < ke) sum(kb);
+  if constexpr (PARTS) {
+    if (!part) {   // (all but the last part are whole slabs: the pointers stand at the next one's first)
+      acc_t total[2][2];
+#pragma unroll 1
+      for (int64_t k1 = kb + kper; k1 < k; k1 += kper) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) {
+            total[x][y] = acc[x][y];
+            acc[x][y] = acc_t{T(0), T(0), T(0), T(0)};
+          }
+        ke = k1 + kper < k ? k1 + kper : k;
+        sum(k1);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) acc[x][y] = total[x][y] + acc[x][y];
+      }
     }
   }
   T* const out = part ? part + (int64_t)blockIdx.y * m * n : C;
@@ -224,10 +258,7 @@ gemm_small_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict_
         const int64_t j = col0 + wn * 32 + 16 * y + Mfma<T>::col(lk, r);
         if (!c_ok(i, j)) continue;
         T v = acc[x][y][r];
-        if (!part && !cinit) {
-          v = alpha * v;
-          v = beta == T(0) ? v : (beta == T(1) ? cv[y][r] + v : beta * cv[y][r] + v);
-        }
+        if (!part && !cinit) v = scaled_sum(v, alpha, beta, cv[y][r]);
         out[i + j * ldo] = v;
       }
   }
@@ -243,8 +274,7 @@ splitk_sum_kernel(int64_t m, int64_t n, int nz, const T* __restrict__ part, T al
   T s = part[i + j * m];
   for (int z = 1; z < nz; ++z) s += part[((int64_t)z * n + j) * m + i];
   T* const c = C + i + j * ldc;
-  const T v = alpha * s;
-  *c = beta == T(0) ? v : (beta == T(1) ? *c + v : beta * *c + v);
+  *c = scaled_sum(s, alpha, beta, beta == T(0) ? T(0) : *c);
 }
 
 // ---- 128 x 128 tiles with the operand slabs moved global -> LDS by the load unit
@@ -530,20 +560,27 @@ static bool small_tiles(int64_t t128, int64_t t64) {
   return (r128 == 1 ? one : more * r128) > 100 * r64;
 }
 
+// nz > 1: k in nz parts, over workgroups with their sums in `part`, or (no `part`) one
+// after the other.
 template <typename T>
 static void small_gemm(bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda, const T* b,
                        int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int64_t tiles, int64_t tri_tiles,
                        int nz, T* part) {
   const int64_t slabs = (k + BK - 1) / BK, kper = (slabs + nz - 1) / nz * BK;
-  const dim3 grid((unsigned)tiles, (unsigned)nz), block(NT);
+  const dim3 grid((unsigned)tiles, part ? (unsigned)nz : 1u), block(NT);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tri, tri_tiles, kper,
                        part);
   };
-  if (!ta && !tb) go(gemm_small_kernel<T, false, false>);
-  else if (ta && !tb) go(gemm_small_kernel<T, true, false>);
-  else if (!ta && tb) go(gemm_small_kernel<T, false, true>);
-  else go(gemm_small_kernel<T, true, true>);
+  auto form = [&](auto parts) {
+    constexpr bool P = decltype(parts)::value;
+    if (!ta && !tb) go(gemm_small_kernel<T, false, false, P>);
+    else if (ta && !tb) go(gemm_small_kernel<T, true, false, P>);
+    else if (!ta && tb) go(gemm_small_kernel<T, false, true, P>);
+    else go(gemm_small_kernel<T, true, true, P>);
+  };
+  if (nz > 1) form(std::true_type{});
+  else form(std::false_type{});
   ZH_LAUNCH_CHECK();
   if (part) {
     hipLaunchKernelGGL(splitk_sum_kernel<T>, dim3((unsigned)((m + 255) / 256), (unsigned)n), dim3(256), 0, s, m, n, nz,
@@ -593,25 +630,18 @@ void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, c
     dma_gemm<T>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, tiles, tri_tiles, 1);
     return;
   }
-  // k is split where the tiles leave CUs idle: about two workgroups per CU, each
-  // with at least 128 of k (a split of 4 or 8 slabs no longer pays its sum)
+  // k is cut into parts where the tiles leave CUs idle: about two workgroups per CU,
+  // each with at least 128 of k (parts of 4 or 8 slabs no longer pay their sum). The
+  // parts follow from the shape alone, so that a product recorded into a graph, where
+  // they have no memory, has the direct one's bits. Their sums (nz m n values: at most
+  // two tiles per CU, a triangle's up to four) go to a workspace of one size: it never
+  // grows, which would wait for the device.
+  const int64_t cus = device_cu_count();
   int nz = 1;
-  if (split_slot >= 0 && stiles < device_cu_count())
-    nz = (int)std::max<int64_t>(1, std::min<int64_t>({2 * device_cu_count() / stiles, k / 128, 32}));
+  if (split_slot >= 0 && stiles < cus)
+    nz = (int)std::max<int64_t>(1, std::min<int64_t>({2 * cus / stiles, k / 128, 32}));
   T* part = nullptr;
-  if (nz > 1) {
-    // the partial sums (at most 2 x CUs tiles) need a workspace: without one (no
-    // memory, or a stream under capture, where nothing may be allocated) no split
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
-      try {
-        part = static_cast<T*>(workspace(sizeof(T) * (size_t)nz * m * n, split_slot));
-      } catch (const HipError&) {
-        (void)hipGetLastError();
-      }
-    }
-    if (!part) nz = 1;
-  }
+  if (nz > 1) part = static_cast<T*>(try_workspace(sizeof(double) * 4 * (size_t)cus * SM * SM, split_slot, s));
   small_gemm<T>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, stiles, stri, nz, part);
 }
 template void gemm_cm<double>(int, int, int64_t, int64_t, int64_t, double, const double*, int64_t, const double*,

@@ -33,9 +33,20 @@ struct DeviceState {
   hipEvent_t fence = nullptr;   // end of the previous call of this thread on this device
   bool fence_set = false;
 };
+// While it lives, this thread's allocations and frees do not end a capture that
+// another thread has under way.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  ~RelaxedCapture() {
+    if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
 struct ThreadState {
   std::unordered_map<int, DeviceState> dev;
   ~ThreadState() {
+    if (dev.empty()) return;
+    const RelaxedCapture relaxed;
     for (auto& kv : dev) {
       int cur = 0;
       if (hipGetDevice(&cur) != hipSuccess) continue;
@@ -135,6 +146,23 @@ void* workspace(size_t bytes, int slot) {
     b.bytes = sz;
   }
   return b.ptr;
+}
+
+void* try_workspace(size_t bytes, int slot, hipStream_t s) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  DeviceState& ds = current();
+  if (ds.slot[slot].bytes >= bytes) return ds.slot[slot].ptr;
+  const RelaxedCapture relaxed;
+  try {
+    return workspace(bytes, slot);
+  } catch (const HipError&) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
 }
 
 // A call on host memory takes two to four blocks; allocating and freeing them cost

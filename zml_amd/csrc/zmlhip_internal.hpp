@@ -84,6 +84,10 @@ const char* last_error();
 // Growable device workspace owned by the library, one per (thread, device).
 // Handed-out pointers stay valid until the next ensure() with a larger size.
 void* workspace(size_t bytes, int slot = 0);
+// The same for work on stream s that can do without: nullptr while s is under capture
+// (memory that a graph uses would be shared with later calls) or when there is no
+// memory. Captures of other threads are not disturbed.
+void* try_workspace(size_t bytes, int slot, hipStream_t s);
 
 // Stream used by the synchronous host-pointer entry points of this thread.
 hipStream_t host_api_stream();
@@ -147,8 +151,8 @@ inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // Element-type generic forms (T = double or float) of the column-major
 // kernels below; the _f64 names are their FP64 instances. split_slot >= 0 allows
-// gemm_cm to split a long k of a small product over workgroups, with the partial
-// sums in that workspace slot (entry points only: a slot serves one stream).
+// gemm_cm to cut a long k of a small product into parts, over workgroups where the
+// partial sums' workspace slot can be had (entry points only: a slot serves one stream).
 template <typename T>
 void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda,
              const T* b, int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int split_slot = -1);
