@@ -290,22 +290,27 @@ trsm_strip_kernel(int q, const T* __restrict__ a, int64_t rs, int64_t cs, T* __r
         else
           fine = fine && ax < T(INFINITY);
       }
-      if (!__all(fine)) {   // the same steps, each vector on one lane
-        if (lr == 0) {
-          for (int k = 0; k < DB; ++k) {
-            T xk = xv[k * XLD];
-            if (MODE != MODE_UNIT) {
-              const T d = i * DB + k < q ? a[(int64_t)(i * DB + k) * (rs + cs)] : T(1);
-              xk = MODE == MODE_DIV ? xk / d : xk * (T(1) / d);
-            }
-            xv[k * XLD] = xk;
-            for (int r = k + 1; r < DB; ++r) xv[r * XLD] = xv[r * XLD] - xk * D[k * DLD + r];
+      if (!__all(fine)) {
+        // the same steps from the start, masked and with exact quotients (the vectors of
+        // this wave alone; 512 rows x 16 vectors 154 us against 75 us on the fast path, and
+        // 1,030 us with each vector on one lane)
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) x[ii] = xv[(lr + 16 * ii) * XLD];
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) {
+#pragma unroll 1
+          for (int kk = 0; kk < 16; ++kk) {
+            const T* const dk = D + (16 * ii + kk) * DLD + lr;
+            const T y = MODE == MODE_DIV ? x[ii] / dg[ii] : (MODE == MODE_MUL ? x[ii] * rinv[ii] : x[ii]);
+            const T xk = __shfl(y, kk, 16);
+            x[ii] = lr == kk ? xk : (lr > kk ? x[ii] - xk * dk[16 * ii] : x[ii]);
+#pragma unroll
+            for (int i2 = ii + 1; i2 < 4; ++i2) x[i2] = x[i2] - xk * dk[16 * i2];
           }
         }
-      } else {
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) xv[(lr + 16 * ii) * XLD] = x[ii];
       }
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) xv[(lr + 16 * ii) * XLD] = x[ii];
     }
     __syncthreads();
     // the solved rows to memory, along B's contiguous direction
