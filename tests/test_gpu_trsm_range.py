@@ -52,7 +52,7 @@ def system(kind, q, nvec, dtype, rng):
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("mode", ["div", "mul", "unit"])
-@pytest.mark.parametrize("q", [1, 2, 15, 16, 17, 32, 33, 48, 49, 63, 64])
+@pytest.mark.parametrize("q", [1, 2, 7, 8, 9, 15, 16, 17, 32, 33, 48, 49, 63, 64])
 def test_bits_of_the_plain_substitution(zh, kind, dtype, mode, q):
     nvec = 21
     rng = np.random.default_rng(q + 100 * KINDS.index(kind))

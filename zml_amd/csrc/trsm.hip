@@ -276,10 +276,13 @@ trsm_strip_kernel(int q, const T* __restrict__ a, int64_t rs, int64_t cs, T* __r
           fine = fine && ad > T(0x1p-400) && ad < T(0x1p+400);
         }
       }
+      // (groups past the last row are the identity's: 16 rows 18.1 us with their steps,
+      // 17.0 without)
+      const int left = q - i * DB;
       strip_group<T, MODE, 0>(x, dd, dg, rinv, D, lr);
-      strip_group<T, MODE, 1>(x, dd, dg, rinv, D, lr);
-      strip_group<T, MODE, 2>(x, dd, dg, rinv, D, lr);
-      strip_group<T, MODE, 3>(x, dd, dg, rinv, D, lr);
+      if (__builtin_expect(left > 16, 1)) strip_group<T, MODE, 1>(x, dd, dg, rinv, D, lr);
+      if (__builtin_expect(left > 32, 1)) strip_group<T, MODE, 2>(x, dd, dg, rinv, D, lr);
+      if (__builtin_expect(left > 48, 1)) strip_group<T, MODE, 3>(x, dd, dg, rinv, D, lr);
       // infinities and NaN (which the unmasked steps would carry to every row),
       // and for the quotients anything near the ends of the range
 #pragma unroll
@@ -290,7 +293,7 @@ trsm_strip_kernel(int q, const T* __restrict__ a, int64_t rs, int64_t cs, T* __r
         else
           fine = fine && ax < T(INFINITY);
       }
-      if (!__all(fine)) {
+      if (__builtin_expect(!__all(fine), 0)) {
         // the same steps from the start, masked and with exact quotients (the vectors of
         // this wave alone; 512 rows x 16 vectors 154 us against 75 us on the fast path, and
         // 1,030 us with each vector on one lane)
@@ -390,6 +393,37 @@ trsm_update_kernel(int64_t m, int K, const T* __restrict__ a, int64_t rs, int64_
     }
 }
 
+// At most FEW rows: one vector per thread, M in scalar registers. Bound by the launch
+// and one round trip to memory: 13.2 us for 4 and 13.3 us for 8 rows, launch included,
+// where the strip's block of 64 rows takes 17.1 and 16.7 us (2 to 1,000 vectors; 16
+// rows 17.0 us on the strip, 64 rows 16.8).
+constexpr int FEW = 8;
+template <typename T>
+__global__ void __launch_bounds__(64)
+trsm_few_kernel(int q, int mode, const T* __restrict__ a, int64_t rs, int64_t cs, T* __restrict__ b, int64_t bs,
+                int64_t vs, int64_t nvec) {
+#pragma clang fp contract(off)
+  const int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (v >= nvec) return;
+  b += v * vs;
+  T m[FEW][FEW], x[FEW];   // rows from q on: row q - 1 again, not stored
+#pragma unroll
+  for (int r = 0; r < FEW; ++r) {
+#pragma unroll
+    for (int c = 0; c <= r; ++c) m[r][c] = a[min(r, q - 1) * rs + min(c, q - 1) * cs];
+    x[r] = b[min(r, q - 1) * bs];
+  }
+#pragma unroll
+  for (int k = 0; k < FEW; ++k) {
+    if (k >= q) break;
+    if (mode == MODE_DIV) x[k] = x[k] / m[k][k];
+    else if (mode == MODE_MUL) x[k] = x[k] * (T(1) / m[k][k]);
+    b[k * bs] = x[k];
+#pragma unroll
+    for (int i = k + 1; i < FEW; ++i) x[i] = x[i] - x[k] * m[i][k];
+  }
+}
+
 template <typename T>
 size_t strip_lds(int64_t q) {
   return sizeof(T) * ((size_t)DB * DLD + (size_t)((q + DB - 1) / DB * DB) * XLD);
@@ -442,6 +476,12 @@ void trsm_cm(int side, int uplo, int transa, int diag, int64_t m, int64_t n, T a
     a0 += (q - 1) * (rs + cs);
     b0 += (q - 1) * bs;
     rs = -rs; cs = -cs; bs = -bs;
+  }
+  if (q <= FEW) {
+    hipLaunchKernelGGL(trsm_few_kernel<T>, dim3((unsigned)((nvec + 63) / 64)), dim3(64), 0, s, (int)q, mode, a0, rs, cs,
+                       b0, bs, vs, nvec);
+    ZH_LAUNCH_CHECK();
+    return;
   }
   for (int64_t i0 = 0; i0 < q; i0 += QB) {
     const int64_t kb = std::min<int64_t>(QB, q - i0), i1 = i0 + kb, rest = q - i1;
