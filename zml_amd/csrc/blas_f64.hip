@@ -120,6 +120,40 @@ laswp_kernel(int64_t ncols, double* __restrict__ a, int64_t sr, int64_t sc, int 
   }
 }
 
+// The same with one thread per column, which makes the exchanges one after the other.
+__global__ void __launch_bounds__(256)
+laswp_each_kernel(int64_t ncols, double* __restrict__ a, int64_t sr, int64_t sc, int k1, int k2,
+                  const int32_t* __restrict__ ipiv, int inc, int ix0, int incx) {
+  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (c >= ncols) return;
+  a += c * sc;
+  const int steps = inc > 0 ? k2 - k1 + 1 : k1 - k2 + 1;
+  for (int s = 0; s < steps; ++s) {
+    const int i = k1 + inc * s, ip = ipiv[ix0 + (int64_t)s * incx] - 1;
+    if (i < 0 || ip < 0 || ip == i) continue;   // (an entry below 1 names no row)
+    double* const p = a + (int64_t)i * sr;
+    double* const q = a + (int64_t)ip * sr;
+    const double t = *p;
+    *p = *q;
+    *q = t;
+  }
+}
+// Whether that one is the faster: its exchanges cost 0.18 us each (0.33 us once the
+// rows no longer fit the L2s) whatever the number of columns, until memory limits it,
+// while the composed moves pay their composition in every workgroup of 8 columns and,
+// along a row, half a cache line a move. Rows contiguous, composed against each:
+// 4 interchanges x 100,000 columns 87 / 14 us, 16 x 500 15.7 / 17.0 and x 4,000 16.3 /
+// 14.8, 64 x 4,000 20.8 / 23.5 and x 8,000 28.7 / 23.9, 256 x 4,000 58 / 58 and x
+// 8,000 80 / 70, 512 x 8,000 115 / 180 and x 16,000 203 / 180, 1,024 x 16,000 351 / 334
+// and x 100,000 1,756 / 761, 4,000 x 16,000 1,432 / 1,847 and x 60,000 4,177 / 2,509. Columns contiguous: 4 x 2,000 14.6 / 14.8, 16 x 8,000 19.9 / 23.9
+// and x 16,000 27.8 / 24.4, 64 x 30,000 68 / 76 and x 60,000 120 / 100, 256 x
+// 100,000 470 / 1,030.
+static bool laswp_each(int64_t ncols, int64_t steps, bool rows_contiguous) {
+  if (steps <= 8) return true;   // 4 x 64: 14.8 / 12.1 us
+  if (!rows_contiguous) return ncols >= 700 * steps;
+  return ncols >= std::min<int64_t>(64 * steps, steps <= 256 ? 5000 : steps <= 1024 ? 14000 : 30000);
+}
+
 constexpr int TT = 32;   // transpose tile
 
 template <typename T>
@@ -193,8 +227,12 @@ static void laswp(int64_t ncols, double* a, int64_t sr, int64_t sc, int k1, int 
                   hipStream_t s, int ix0, int incx) {
   if (ncols <= 0) return;
   if (ix0 < 0) { ix0 = k1; incx = inc; }   // the interchange of row k uses ipiv[k], in both orders
-  hipLaunchKernelGGL(laswp_kernel, dim3((unsigned)((ncols + LW_CB - 1) / LW_CB)), dim3(2 * LW_NS), 0, s, ncols, a, sr,
-                     sc, k1, k2, ipiv, inc, ix0, incx);
+  if (laswp_each(ncols, (int64_t)(inc > 0 ? k2 - k1 : k1 - k2) + 1, sc == 1))
+    hipLaunchKernelGGL(laswp_each_kernel, dim3((unsigned)((ncols + 255) / 256)), dim3(256), 0, s, ncols, a, sr, sc, k1,
+                       k2, ipiv, inc, ix0, incx);
+  else
+    hipLaunchKernelGGL(laswp_kernel, dim3((unsigned)((ncols + LW_CB - 1) / LW_CB)), dim3(2 * LW_NS), 0, s, ncols, a, sr,
+                       sc, k1, k2, ipiv, inc, ix0, incx);
   ZH_LAUNCH_CHECK();
 }
 void laswp_rm(int64_t ncols, double* a, int64_t lda, int k1, int k2, const int32_t* ipiv, int inc,
