@@ -552,16 +552,19 @@ template void scale_cm<float>(int64_t, int64_t, float, float*, int64_t, hipStrea
 // 2512 609 against 671 us. FP32: 2048 x 2176 x 768 117 against 91 us, 2048^3 186
 // against 190 us, 2500^2 x 2496 349 against 386 us, 3100 x 2900 x 3008 (575 tiles)
 // 664 against 581 us, 4096^3 1127 against 1362 us.
+// In FP32, up to k = 128, four workgroups a CU hide the operands' first slab and the
+// reads and writes of C, which the larger tiles' two do not: 6000^2 x 64 117 against
+// 86 us, 5000^2 x 128 124 against 98, 12000^2 x 128 527 against 462. Beyond it depends on
+// the form: k = 192 5000^2 154 against 130 us, 8192^2 333 against 354.
 template <typename T>
-static bool small_tiles(int64_t t128, int64_t t64) {
+static bool small_tiles(int64_t t128, int64_t t64, int64_t k) {
+  if (sizeof(T) == 4 && k <= 128) return true;
   const int64_t cus = device_cu_count();
   const int64_t r128 = (t128 + cus - 1) / cus, r64 = (t64 + cus - 1) / cus;
   constexpr int one = sizeof(T) == 8 ? 364 : 400, more = sizeof(T) == 8 ? 326 : 345;
   return (r128 == 1 ? one : more * r128) > 100 * r64;
 }
 
-// nz > 1: k in nz parts, over workgroups with their sums in `part`, or (no `part`) one
-// after the other.
 template <typename T>
 static void small_gemm(bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alpha, const T* a, int64_t lda, const T* b,
                        int64_t ldb, T beta, T* c, int64_t ldc, hipStream_t s, int tri, int64_t tiles, int64_t tri_tiles,
@@ -626,7 +629,7 @@ void gemm_cm(int transa, int transb, int64_t m, int64_t n, int64_t k, T alpha, c
   const int64_t tiles = tri_tiles > 0 ? tri_tiles : ntm * ntn;
   const int64_t nsm = (m + SM - 1) / SM, nsn = (n + SM - 1) / SM;
   const int64_t stri = tri_tile_count(tri, nsm, nsn), stiles = stri > 0 ? stri : nsm * nsn;
-  if (gemm_dma_enabled() && dma_ok<T>(ta, tb, m, n, k, a, lda, b, ldb) && !small_tiles<T>(tiles, stiles)) {
+  if (gemm_dma_enabled() && dma_ok<T>(ta, tb, m, n, k, a, lda, b, ldb) && !small_tiles<T>(tiles, stiles, k)) {
     dma_gemm<T>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, tiles, tri_tiles, 1);
     return;
   }
