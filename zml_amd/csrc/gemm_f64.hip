@@ -100,7 +100,7 @@ __device__ __forceinline__ void tile_coords(int64_t bid, int64_t ntm, int64_t nt
 // 67 us, 124 x 918 x 5130 (k split 17 ways) 838 -> 43 us.
 constexpr int SM = 64, SLD = SM + 2;
 
-// The last rounding steps of a product whose sum is s.
+// The last rounding steps of a product in parts whose sum is s, the same in both kernels.
 template <typename T>
 __device__ __forceinline__ T scaled_sum(T s, T alpha, T beta, T c) {
 #pragma clang fp contract(off)
@@ -258,7 +258,12 @@ gemm_small_kernel(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict_
         const int64_t j = col0 + wn * 32 + 16 * y + Mfma<T>::col(lk, r);
         if (!c_ok(i, j)) continue;
         T v = acc[x][y][r];
-        if (!part && !cinit) v = scaled_sum(v, alpha, beta, cv[y][r]);
+        if constexpr (PARTS) {
+          if (!part) v = scaled_sum(v, alpha, beta, cv[y][r]);
+        } else if (!cinit) {
+          v = alpha * v;
+          v = beta == T(0) ? v : (beta == T(1) ? cv[y][r] + v : beta * cv[y][r] + v);
+        }
         out[i + j * ldo] = v;
       }
   }
