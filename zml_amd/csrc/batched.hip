@@ -857,10 +857,10 @@ BatchPlan* batch_plan_create(int count, const int* n, const int* nrhs, const int
     P->bucket_count[bk] = (int)lists[bk].size();
     flat.insert(flat.end(), lists[bk].begin(), lists[bk].end());
   }
-  ZH_CHECK(hipMalloc(&P->d_sys, sizeof(SysDesc) * std::max(count, 1)));
-  ZH_CHECK(hipMalloc(&P->d_lists, sizeof(int) * std::max<size_t>(flat.size(), 1)));
-  ZH_CHECK(hipMalloc(&P->d_counters, sizeof(int) * 64));
-  ZH_CHECK(hipMalloc(&P->d_status, sizeof(int) * std::max(count, 1)));
+  ZH_CHECK(device_alloc(reinterpret_cast<void**>(&P->d_sys), sizeof(SysDesc) * std::max(count, 1)));
+  ZH_CHECK(device_alloc(reinterpret_cast<void**>(&P->d_lists), sizeof(int) * std::max<size_t>(flat.size(), 1)));
+  ZH_CHECK(device_alloc(reinterpret_cast<void**>(&P->d_counters), sizeof(int) * 64));
+  ZH_CHECK(device_alloc(reinterpret_cast<void**>(&P->d_status), sizeof(int) * std::max(count, 1)));
   ZH_CHECK(hipMemcpyAsync(P->d_sys, h.data(), sizeof(SysDesc) * count, hipMemcpyHostToDevice, s));
   if (!flat.empty())
     ZH_CHECK(hipMemcpyAsync(P->d_lists, flat.data(), sizeof(int) * flat.size(), hipMemcpyHostToDevice, s));

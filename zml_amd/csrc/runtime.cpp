@@ -124,6 +124,19 @@ void profile_collect(int kind, double* ms, long long* launches, double* flops, d
 }
 const char* last_error() { return tl_last_error.c_str(); }
 
+hipError_t device_alloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  std::vector<Buf>& kept = current().kept;
+  if (e == hipErrorOutOfMemory && !kept.empty()) {
+    (void)hipGetLastError();
+    for (auto& b : kept) (void)hipFree(b.ptr);
+    kept.clear();
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) (void)hipGetLastError();   // (the next launch check would report it again)
+  return e;
+}
+
 void* workspace(size_t bytes, int slot) {
   if (slot < 0 || slot >= kSlots) throw std::runtime_error("workspace: slot out of range");
   DeviceState& ds = current();
@@ -138,7 +151,7 @@ void* workspace(size_t bytes, int slot) {
       b.bytes = 0;
     }
     size_t sz = align_up(bytes, 1 << 20);
-    hipError_t e = hipMalloc(&b.ptr, sz);
+    hipError_t e = device_alloc(&b.ptr, sz);
     if (e != hipSuccess) {
       b.ptr = nullptr;
       throw HipError(e, "workspace allocation failed");
@@ -167,8 +180,9 @@ void* try_workspace(size_t bytes, int slot, hipStream_t s) {
 
 // A call on host memory takes two to four blocks; allocating and freeing them cost
 // 65 of the 555 us of a 200 x 200 solve (a free waits for the device). Blocks of up to
-// 16 MiB are kept, at most eight per thread and device: above that a call's copies
-// take milliseconds and the allocation no longer shows.
+// 16 MiB are kept, at most eight per thread and device, a larger one in place of the
+// smallest: above that a call's copies take milliseconds and the allocation no longer
+// shows.
 constexpr size_t kKeptBlock = size_t(16) << 20;
 constexpr size_t kKeptBlocks = 8;
 
@@ -185,14 +199,7 @@ void* host_block(size_t bytes, size_t* got) {
   }
   void* p = nullptr;
   *got = bytes <= kKeptBlock ? align_up(bytes, 1 << 16) : bytes;
-  hipError_t e = hipMalloc(&p, *got);
-  if (e == hipErrorOutOfMemory && !kept.empty()) {
-    (void)hipGetLastError();
-    for (auto& b : kept) (void)hipFree(b.ptr);
-    kept.clear();
-    e = hipMalloc(&p, *got);
-  }
-  ZH_CHECK(e);
+  ZH_CHECK(device_alloc(&p, *got));
   return p;
 }
 
@@ -201,13 +208,16 @@ void host_block_done(void* p, size_t got, bool keep) noexcept {
   if (keep && got <= kKeptBlock) {
     try {
       std::vector<Buf>& kept = current().kept;
+      Buf b;
+      b.ptr = p;
+      b.bytes = got;
       if (kept.size() < kKeptBlocks) {
-        Buf b;
-        b.ptr = p;
-        b.bytes = got;
         kept.push_back(b);
         return;
       }
+      for (auto& k : kept)
+        if (k.bytes < b.bytes) std::swap(k, b);   // leaves the smallest in b
+      p = b.ptr;
     } catch (...) {
     }
   }

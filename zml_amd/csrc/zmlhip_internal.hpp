@@ -81,6 +81,10 @@ struct SyncError : std::runtime_error {
 void set_last_error(const std::string& msg);
 const char* last_error();
 
+// hipMalloc; when there is no memory, after giving this thread's idle host_block
+// memory back.
+hipError_t device_alloc(void** p, size_t bytes);
+
 // Growable device workspace owned by the library, one per (thread, device).
 // Handed-out pointers stay valid until the next ensure() with a larger size.
 void* workspace(size_t bytes, int slot = 0);
