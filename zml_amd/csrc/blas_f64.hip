@@ -145,9 +145,9 @@ laswp_each_kernel(int64_t ncols, double* __restrict__ a, int64_t sr, int64_t sc,
 // 4 interchanges x 100,000 columns 87 / 14 us, 16 x 500 15.7 / 17.0 and x 4,000 16.3 /
 // 14.8, 64 x 4,000 20.8 / 23.5 and x 8,000 28.7 / 23.9, 256 x 4,000 58 / 58 and x
 // 8,000 80 / 70, 512 x 8,000 115 / 180 and x 16,000 203 / 180, 1,024 x 16,000 351 / 334
-// and x 100,000 1,756 / 761, 4,000 x 16,000 1,432 / 1,847 and x 60,000 4,177 / 2,509. Columns contiguous: 4 x 2,000 14.6 / 14.8, 16 x 8,000 19.9 / 23.9
-// and x 16,000 27.8 / 24.4, 64 x 30,000 68 / 76 and x 60,000 120 / 100, 256 x
-// 100,000 470 / 1,030.
+// and x 100,000 1,756 / 761, 4,000 x 16,000 1,432 / 1,847 and x 60,000 4,177 / 2,509.
+// Columns contiguous: 4 x 2,000 14.6 / 14.8, 16 x 8,000 19.9 / 23.9 and x 16,000 27.8 /
+// 24.4, 64 x 30,000 68 / 76 and x 60,000 120 / 100, 256 x 100,000 470 / 1,030.
 static bool laswp_each(int64_t ncols, int64_t steps, bool rows_contiguous) {
   if (steps <= 8) return true;   // 4 x 64: 14.8 / 12.1 us
   if (!rows_contiguous) return ncols >= 700 * steps;

@@ -505,12 +505,6 @@ static const int32_t* fused_block_perm(int64_t j0) {
   return tl_fused[dev & 15].pairs[(j0 / NB_F64) & 1];
 }
 
-// The share of a trailing update to apply beside the next panel (on the CUs
-// the panel leaves free): a fixed 5 ms of update on 192 CUs at 44 TF/s, the
-// rest then runs on all 256 CUs once the panel is done. (Measured on one
-// MI355X at n = 32768: 718 ms per LU; sizing it to the one-launch panel's
-// 7.4 ms plus 20% gave 729 ms.)
-
 // Plain partial-pivoting LU of a row-major matrix in T (FP64 for dgetrf, FP32
 // for sgetrf): the same driver, leaves and kernels, no low-precision update.
 // FP64 factors each block column in one launch (panel_fused.hpp).
@@ -523,12 +517,14 @@ void getrf_rm(int64_t m, int64_t n, T* A, int64_t lda, int32_t* ipiv, int* info,
   // of the CUs, those CUs are kept free of trailing updates so the panel never
   // waits for GEMM tiles to drain (rounded up to a power of two from 8, so few
   // distinct masked streams exist).
-  // The height threshold (panel_one_launch_rows, default 16384): measured per
-  // panel height on one MI355X, the one-launch panel wins above 16384 rows
-  // (where the leaf's 256-row grid no longer fits the reserved CUs) and loses
-  // below (n = 16384: 242 ms against 172 ms), its in-kernel update of the
-  // block column being slower than the MFMA GEMMs the leaf path launches
-  // between leaves.
+  // The height threshold (panel_one_launch_rows, default 16384): above it the
+  // leaves' 256-row workgroups are more than the 64 CUs kept free, so that a leaf
+  // waits for trailing-update tiles to drain, while the one-launch panel's 512-row
+  // ones fit up to 32768 rows: n = 17000 112 ms against 130 leaf by leaf, 24576 270
+  // against 293, 32768 569 against 594. Below, the leaves have their CUs too and the
+  // MFMA GEMMs between them are faster than the panel's own update of its block
+  // column (512 columns alone: 2.2 ms at 16384 rows against 6.7): n = 16384 104 ms
+  // against 153 with the line at 8192.
   const int64_t kFusedMinRows = panel_one_launch_rows();
   const int64_t first_rows = sizeof(T) == 8 && m > kFusedMinRows ? panel::FPT : panel::pt_of<T>();
   const int leaf_wgs = (int)((m + first_rows - 1) / first_rows);

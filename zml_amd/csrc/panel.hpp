@@ -193,8 +193,8 @@ __device__ __forceinline__ void update_row(T (&a)[W], T l, const T* __restrict__
 // Leaf LU: rows [0, M) x columns [0, Wn) of the row-major panel P (Wn <= 64).
 // ipiv[k] = piv_base + pivot row + 1 (1-based, global); *info gets
 // info_base + first zero pivot (1-based) when it is still 0.
-// For more than one workgroup, which exchange through ws (panels of up to 1,024
-// rows take the one-workgroup leaf of panel_leaf1.hpp).
+// For panels of more than 512 rows, whose workgroups exchange through ws, with the
+// look-ahead switch off (panel_leaf1.hpp has the others').
 // A wait that exceeds spin_limit polls (or any wait, when spin_limit < 0)
 // sets *ws.err and ends the kernel in every workgroup; the factors are then
 // invalid and the host reports the give-up.

@@ -41,7 +41,8 @@ constexpr int DB = 128;   // diagonal block of the driver
 // Each element receives its separately rounded updates a - l_ik l_ck in the order
 // of k, as in the unblocked right-looking algorithm: the same bits as one column
 // at a time over the whole block, which spent its time on masks and on one
-// barrier per column (158 us per 128 x 128 block on MI355X, against 42 us). Bound by
+// barrier per column (158 us per 128 x 128 block alone on MI355X, against 42 us; 97 to
+// 133 us inside a factorization, beside the trailing update's workgroups). Bound by
 // the step chain of one wave (310 cycles a column: square root, reciprocal, up to
 // 15 readlane pairs with their multiplies and subtracts), then by the later
 // columns' updates (230 cycles a column on average).
