@@ -517,19 +517,21 @@ __global__ void __launch_bounds__((ND + ND / 2) * 64, ND == 8 ? 3 : 4) batched_t
           sh.xv[u][q] = x[q];
         }
         __syncthreads();   // R3
-        // r = b - A x and the row sums of |A|, one row per thread, columns in order
-        double acc[BQ], asum = 0.0;
+        // r = b - A x and the row sums of |A|, one row per thread: sums of 8 columns,
+        // added up (one column after the other onto b left solutions 1.8 to 2.4 times as far
+        // from the exact ones: 4.6e-16 against 2.5e-16 at n = 70, 1.16e-15 against 4.7e-16 at 256)
+        double acc[BQ], sum[BQ], asum = 0.0;
 #pragma unroll
-        for (int q = 0; q < BQ; ++q) acc[q] = q < nq && u < n ? b[(int64_t)q * n + u] : 0.0;
+        for (int q = 0; q < BQ; ++q) sum[q] = 0.0;
         if (u < n) {
           const double* pa = d.a + u;
           auto one = [&](double v, int j) __attribute__((always_inline)) {
             const double2 x01 = *reinterpret_cast<const double2*>(&sh.xv[j][0]);
             const double2 x23 = *reinterpret_cast<const double2*>(&sh.xv[j][2]);
-            acc[0] -= v * x01.x;
-            acc[1] -= v * x01.y;
-            acc[2] -= v * x23.x;
-            acc[3] -= v * x23.y;
+            acc[0] += v * x01.x;
+            acc[1] += v * x01.y;
+            acc[2] += v * x23.x;
+            acc[3] += v * x23.y;
             asum += fabs(v);
           };
           int j = 0;
@@ -538,10 +540,23 @@ __global__ void __launch_bounds__((ND + ND / 2) * 64, ND == 8 ? 3 : 4) batched_t
 #pragma unroll
             for (int e = 0; e < 16; ++e) v[e] = pa[(int64_t)(j + e) * n];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) one(v[e], j + e);
+            for (int h = 0; h < 16; h += 8) {
+#pragma unroll
+              for (int q = 0; q < BQ; ++q) acc[q] = 0.0;
+#pragma unroll
+              for (int e = h; e < h + 8; ++e) one(v[e], j + e);
+#pragma unroll
+              for (int q = 0; q < BQ; ++q) sum[q] += acc[q];
+            }
           }
+#pragma unroll
+          for (int q = 0; q < BQ; ++q) acc[q] = 0.0;
           for (; j < n; ++j) one(pa[(int64_t)j * n], j);
+#pragma unroll
+          for (int q = 0; q < BQ; ++q) sum[q] += acc[q];
         }
+#pragma unroll
+        for (int q = 0; q < BQ; ++q) acc[q] = q < nq && u < n ? b[(int64_t)q * n + u] - sum[q] : 0.0;
         double mx[2 * BQ + 1];
 #pragma unroll
         for (int q = 0; q < BQ; ++q) {
