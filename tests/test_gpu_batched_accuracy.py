@@ -74,3 +74,22 @@ def test_errors_of_residuals_summed_in_parts(zh, torch_cuda, n):
     assert np.all(status >= 0)
     E = exact(A, B)
     assert mean_error(X, E) <= 1.15 * mean_error(refined(A, B, 8), E)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [20, 40, 70, 110, 128, 150, 200, 256])
+@pytest.mark.parametrize("decades", [20, 25, 30, 35])
+def test_no_success_without_a_solution(zh, torch_cuda, n, decades):
+    """Columns over up to 70 decades, which the FP32 factors cannot hold: some entries of
+    a solution come out as NaN while others are numbers. Such a system has to say so."""
+    rng = np.random.default_rng(n + decades)
+    c = 10.0 ** rng.uniform(-decades, decades, (20, n))
+    A = (rng.uniform(-1, 1, (20, n, n)) + n / 4.0 * np.eye(n)) * c[:, None, :]
+    B = np.matmul(A, rng.uniform(-1, 1, (20, n, 2)) / c[:, :, None])
+    bt = Batch(zh, torch_cuda, [(a, b, False) for a, b in zip(A, B)], autotune=0)
+    status, hx = bt.run()
+    for k, X in enumerate(bt.solutions(hx)):
+        if status[k] >= 0:
+            R = np.abs(B[k] - A[k] @ X).max(axis=0)
+            assert np.all(R <= 16 * n * 2.0 ** -53 * np.abs(A[k]).sum(1).max() * np.abs(X).max(axis=0))
+    bt.close()

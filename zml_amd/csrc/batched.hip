@@ -271,7 +271,7 @@ __global__ void __launch_bounds__(TY * TX) batched_solve_kernel(BatchArgs g) {
             asum += pabs[q * NMAX + t];
           }
           rv[t] = accd;
-          ri = fabs(accd);
+          ri = accd == accd ? fabs(accd) : INFINITY;   // (a maximum passes over NaN)
           ai = asum;
         }
         if (anorm == 0.0) anorm = block_max<NW>(ai, red, t);
@@ -280,7 +280,7 @@ __global__ void __launch_bounds__(TY * TX) batched_solve_kernel(BatchArgs g) {
         ++it;
         const double be = rmax / (anorm * xmax * (double)n * 0x1p-53);
         if (be <= g.tol) break;
-        if (!(be == be) || it >= g.max_iter || (it >= 2 && be > 0.5 * prev)) {
+        if (!(be < INFINITY) || it >= g.max_iter || (it >= 2 && be > 0.5 * prev)) {
           it = -1;
           break;
         }
@@ -561,7 +561,7 @@ __global__ void __launch_bounds__((ND + ND / 2) * 64, ND == 8 ? 3 : 4) batched_t
 #pragma unroll
         for (int q = 0; q < BQ; ++q) {
           sh.rv[q][u] = acc[q];
-          mx[q] = fabs(acc[q]);
+          mx[q] = acc[q] == acc[q] ? fabs(acc[q]) : INFINITY;   // (a maximum passes over NaN)
           mx[BQ + q] = fabs(x[q]);
         }
         mx[2 * BQ] = asum;
@@ -586,7 +586,7 @@ __global__ void __launch_bounds__((ND + ND / 2) * 64, ND == 8 ? 3 : 4) batched_t
           const double be = mx[q] / (anorm * mx[BQ + q] * (double)n * 0x1p-53);
           if (be <= g.tol) {
             act[q] = false;
-          } else if (!(be == be) || it[q] >= g.max_iter || (it[q] >= 2 && be > 0.5 * prev[q])) {
+          } else if (!(be < INFINITY) || it[q] >= g.max_iter || (it[q] >= 2 && be > 0.5 * prev[q])) {
             it[q] = -1;
             act[q] = false;
           } else {
